@@ -39,6 +39,9 @@ namespace dgops
     T xq[max_n];   // Gauss points on [0,1]
     T xn[max_n]; // Gauss-Lobatto nodes on [0,1]
     EvenOdd<T> eo_S, eo_Sinv, eo_D; // even-odd forms of S, S^-1, D
+    // even and odd parts of l0 and dl0 (l1 is l0 reversed, dl1 is -dl0
+    // reversed) and their middle values: l0 = le + lo, dl0 = de + dd
+    T le[max_h], lo[max_h], de[max_h], dd[max_h], lm, dm;
   };
 
   template <typename T>
@@ -90,6 +93,17 @@ namespace dgops
         d.xq[i]    = (T)b.gauss_pts[i];
         d.xn[i]    = (T)b.gl_pts[i];
       }
+    const int h = b.n / 2;
+    for (int i = 0; i < h; ++i)
+      {
+        const int r = b.n - 1 - i;
+        d.le[i]     = (T)(0.5 * (b.l0[i] + b.l0[r]));
+        d.lo[i]     = (T)(0.5 * (b.l0[i] - b.l0[r]));
+        d.de[i]     = (T)(0.5 * (b.dl0[i] + b.dl0[r]));
+        d.dd[i]     = (T)(0.5 * (b.dl0[i] - b.dl0[r]));
+      }
+    d.lm      = (T)b.l0[h];
+    d.dm      = (T)b.dl0[h];
     d.eo_S    = make_even_odd<T>(b.S, b.n);
     d.eo_Sinv = make_even_odd<T>(b.Sinv, b.n);
     d.eo_D    = make_even_odd<T>(b.D, b.n);

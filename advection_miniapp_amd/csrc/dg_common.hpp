@@ -33,6 +33,7 @@ namespace dgops
     const int    *neighbors;     // [cell][2 dim]
     const double *cell_vertices; // [cell][2^dim][dim]
     double        h[3];          // cell size when `cartesian`
+    double        inv_h[3];      // its reciprocals
     int           cartesian;
     int           vel_kind;
     double        vel_const[3];
@@ -63,6 +64,7 @@ namespace dgops
     const void   *tab_cell;
     const void   *tab_face;
     const double *tab_bnd;
+    int           has_boundary; // the mesh has boundary faces
     const int    *bnd_index; // [cell][2 dim] boundary face id, -1 inside
     const double *bnd_value; // [boundary face][nl] Dirichlet data at sol_time
   };

@@ -251,6 +251,7 @@ namespace dgops
     for (int d = 0; d < 3; ++d)
       {
         P.h[d]         = mesh.h[d];
+        P.inv_h[d]     = 1. / mesh.h[d];
         P.vel_const[d] = cfg.velocity[d];
       }
     P.cartesian = cfg.perturbation == 0.;
@@ -322,6 +323,7 @@ namespace dgops
     Pk.tab_bnd   = m.d_tab_bnd.as<double>();
     Pk.bnd_index = m.d_bnd_index.as<int>();
     Pk.bnd_value = m.d_bnd_value.as<double>();
+    Pk.has_boundary = m.n_bnd > 0;
     aux_boundary_values(m, Pk);
     const uint32_t base = op_key(op.cfg.dim, op.n, nc, fp32 ? 1 : 0,
                                  geo, skew ? 1 : 0, diff, fin, epi);

@@ -310,15 +310,14 @@ namespace dgops
   // a cell read contiguous memory
   template <int dim, int n, typename T>
   __device__ __forceinline__ void
-  table_line(const T *tab, int64_t cell, int row, int p, bool active,
-             T (&v)[n])
+  table_line(const T *tab, int64_t cell, int row, int p, T (&v)[n])
   {
     constexpr int nd   = Lay<dim, n>::nd;
     constexpr int nl   = Lay<dim, n>::nl;
     const T      *base = tab + (cell * (dim + 1) + row) * nd;
 #pragma unroll
     for (int i = 0; i < n; ++i)
-      v[i] = active ? base[i * nl + p] : (T)0;
+      v[i] = base[i * nl + p];
   }
 
   // ---- geometry ------------------------------------------------------------
@@ -392,113 +391,243 @@ namespace dgops
   }
 
 
-  // ---- face terms ------------------------------------------------------------
+  // ---- one direction of the operator -----------------------------------------
 
-  // Numerical flux on the two faces normal to `dir`, at the face point owned
-  // by this thread in the dir-line layout; adds sign * l_side (x) flux to the
-  // line accumulator. Positive-operator convention of
-  // advection_solver_implicit_real.cc:1032-1058:
-  //   F = 1/2 [(u- + u+) an + alpha |an| (u- - u+)] - skew an u-
-  // with an = a . n dA on this cell's outward normal.
-  template <int dim, int n, int dir, typename T, bool diff, bool local = false>
-  __device__ __forceinline__ void
-  face_terms(const OpParams &P,
-             const DevBasis<double> *Bd,
-             const DevBasis<T>      &B,
-             int64_t                 cell,
-             int                     p,
-             bool                    active,
-             const int (&nb)[2 * dim],
-             const T (&uplus)[2 * dim],
-             const T (&dplus)[2 * dim],
-             const T (&uq)[n],
-             T (&acc)[n],
-             T    vf,
-             T (&fan)[2 * dim])
+  // A line of n values in even-odd form: e_i = v_i + v_{n-1-i}, o_i = v_i -
+  // v_{n-1-i} for i < n/2 and the middle value m of odd n.
+  template <int n, typename T>
+  struct EoLine
   {
-    int q[3];
-    Lay<dim, n>::template idx<dir>(p, 0, q);
+    static constexpr int h = n / 2;
+    T                    e[h > 0 ? h : 1], o[h > 0 ? h : 1], m;
+
+    __device__ __forceinline__
+    EoLine(const T (&v)[n])
+    {
 #pragma unroll
-    for (int s = 0; s < 2; ++s)
+      for (int i = 0; i < h; ++i)
+        {
+          e[i] = v[i] + v[n - 1 - i];
+          o[i] = v[i] - v[n - 1 - i];
+        }
+      m = v[h];
+    }
+  };
+
+  // Symmetric part e, antisymmetric part o and middle value m of a line:
+  // v_q = e_q + o_q, v_{n-1-q} = e_q - o_q, v_{n/2} = m.
+  template <int n, typename T>
+  struct EoSum
+  {
+    static constexpr int h = n / 2;
+    T                    e[h > 0 ? h : 1], o[h > 0 ? h : 1], m;
+  };
+
+  // D (transpose: D^T) times the line v; D is skew-centrosymmetric, so the
+  // products with v.e are antisymmetric and those with v.o symmetric (see
+  // eo_apply, which this equals)
+  template <int n, bool transpose, typename T>
+  __device__ __forceinline__ void
+  eo_derivative(const EvenOdd<T> &M, const EoLine<n, T> &v, EoSum<n, T> &r)
+  {
+    constexpr int  h   = n / 2;
+    constexpr bool odd = n % 2 == 1;
+#pragma unroll
+    for (int q = 0; q < h; ++q)
       {
-        const int f = 2 * dir + s;
-        const T(&l)[max_n] = s ? B.l1 : B.l0;
-        T um = l[0] * uq[0];
+        T se = odd ? (transpose ? M.mr[q] : M.mc[q]) * v.m :
+                     (transpose ? M.o[0][q] : M.e[q][0]) * v.e[0];
 #pragma unroll
-        for (int i = 1; i < n; ++i)
-          um = fma(l[i], uq[i], um);
-        T up = uplus[f];
-        if (!local && active && nb[f] < 0)
-          // Dirichlet data, evaluated before the launch
-          // (boundary_value_kernel)
-          up = (T)P.bnd_value[(int64_t)P.bnd_index[cell * 2 * dim + f] *
-                                Lay<dim, n>::nl +
-                              p];
-        const T an = fan[f] * vf;
-        const T flux =
-          (T)0.5 * ((um + up) * an + (T)P.alpha * fabs(an) * (um - up)) -
-          (T)P.skew * an * um;
-        const T sf = (T)P.sign * flux;
+        for (int i = odd ? 0 : 1; i < h; ++i)
+          se = fma(transpose ? M.o[i][q] : M.e[q][i], v.e[i], se);
+        T so = (transpose ? M.e[0][q] : M.o[q][0]) * v.o[0];
 #pragma unroll
-        for (int i = 0; i < n; ++i)
-          acc[i] = fma(l[i], sf, acc[i]);
-        if constexpr (diff)
-          {
-            // SIPG (advection_diffusion_solver.cc:569-613) on this cell's
-            // outward normal, axis-aligned cells: with
-            //   jump = -nu/2 (u- - u+), avg = -nu/2 (d_n u- + d_n u+)
-            // the value term is -(jump sigma - avg) and the normal
-            // derivative of the test function is weighted with jump
-            const T(&dl)[max_n] = s ? B.dl1 : B.dl0;
-            const T hd  = (T)P.h[dir];
-            const T sgn = s ? (T)1 : (T)-1;
-            T       dm  = dl[0] * uq[0];
+        for (int i = 1; i < h; ++i)
+          so = fma(transpose ? M.e[i][q] : M.o[q][i], v.o[i], so);
+        r.e[q] = so;
+        r.o[q] = se;
+      }
+    r.m = 0;
+    if constexpr (odd)
+      {
+        r.m = (transpose ? M.mc[0] : M.mr[0]) * v.o[0];
 #pragma unroll
-            for (int i = 1; i < n; ++i)
-              dm = fma(dl[i], uq[i], dm);
-            const T dnm = sgn * dm / hd, dnp = sgn * dplus[f] / hd;
-            T       w   = (T)1;
-            for (int e = 0; e < dim; ++e)
-              if (e != dir)
-                w *= (T)(Bd->w[q[e]] * P.h[e]);
-            const T nu    = (T)P.viscosity;
-            const T sigma = (T)P.penalty / hd;
-            const T jump  = (T)-0.5 * nu * (um - up);
-            const T avg   = (T)-0.5 * nu * (dnm + dnp);
-            const T fv    = (T)P.sign * w * (avg - jump * sigma);
-            const T fd    = (T)P.sign * w * jump * sgn / hd;
-#pragma unroll
-            for (int i = 0; i < n; ++i)
-              acc[i] = fma(l[i], fv, fma(dl[i], fd, acc[i]));
-          }
+        for (int i = 1; i < h; ++i)
+          r.m = fma(transpose ? M.mc[i] : M.mr[i], v.o[i], r.m);
       }
   }
 
-  // cell diffusion term along direction dir on axis-aligned cells:
-  // acc += D^T (sign nu |K|/h_d^2 w_q D u_q)  (int grad v . nu grad u)
-  template <int dim, int n, int dir, typename T>
-  __device__ __forceinline__ void
-  diffusion_cell_term(const OpParams &P, const DevBasis<double> *Bd,
-                      const DevBasis<T> &B, int p, const T (&uq)[n],
-                      T (&acc)[n])
+  // Per-launch factors of one component's terms, uniform over the grid:
+  // flux = an (c_own u- + c_nb u+) + c_abs |an| (u- - u+) is sign times the
+  // numerical flux 1/2 [(u- + u+) an + alpha |an| (u- - u+)] - skew an u-
+  // (advection_solver_implicit_real.cc:1032-1058, an = a . n dA on the
+  // cell's outward normal) at the speed factor vf.
+  template <typename T>
+  struct FluxFactors
   {
-    double vol = P.h[0] * P.h[1];
-    if (dim == 3)
-      vol *= P.h[2];
-    const T c0 = (T)(P.sign * P.viscosity * vol / (P.h[dir] * P.h[dir]));
-    T       du[n], g[n];
-    eo_apply<n, true, false, false>(B.eo_D, uq, du);
+    T c_own, c_nb, c_abs;
+
+    __device__ __forceinline__
+    FluxFactors(const OpParams &P, double vf)
+      : c_own((T)(P.sign * vf * (0.5 - P.skew)))
+      , c_nb((T)(P.sign * vf * 0.5))
+      , c_abs((T)(P.sign * fabs(vf) * 0.5 * P.alpha))
+    {}
+  };
+
+  // Cell and face terms of direction `dir` on the line owned by this
+  // thread: acc (+)= D^T g + s D u + sum_sides l_side (x) flux, with
+  //   g: the cell flux at the line's points (the caller's, plus the
+  //      diffusion flux cd w_i (D u)_i with `diff`),
+  //   s (skew): the factor of the values' derivative,
+  // and the faces at the line's two ends (fan: a . n dA, up / dp: the
+  // neighbours' traces and reference derivatives normal to the face).
+  // Everything works on even and odd parts: the two end values share their
+  // products (l1 is l0 reversed, the end derivatives change sign), D u and
+  // the end values share the split of u, and the lift of the end values
+  // joins D^T g before the parts are put together. Per line of n points
+  // the faces then cost 2 n products instead of 4 n (4 n instead of 10 n
+  // with diffusion, whose cell flux shares the D^T product of the advective
+  // one), and the reciprocals 1/h come from the launch: these kernels are
+  // bound by VALU issue with diffusion. One MI355X, before and after,
+  // together with the staging of the normal derivatives in the value phase
+  // (FP64 degree 7: 3203 -> 1647 VALU instructions per wave, 236 -> 160
+  // registers): SIPG on 32^3 cells, degree 5 FP64 131 -> 81 us, degree 7
+  // FP32 144 -> 84 us; without diffusion, degree 4 on 64^3 perturbed cells
+  // FP64 375 -> 366 us, degree 6 FP32 on 24^3 cells 32.2 -> 28.0 us.
+  // SIPG (advection_diffusion_solver.cc:569-613) on axis-aligned cells: with
+  // jump = -nu/2 (u- - u+), avg = -nu/2 (d_n u- + d_n u+) the value term is
+  // -(jump sigma - avg) and the normal derivative of the test function is
+  // weighted with jump; wd is the product of the weights of the line's other
+  // coordinates.
+  template <int dim, int n, int dir, typename T, bool skew, bool diff,
+            bool local, bool add>
+  __device__ __forceinline__ void
+  line_operator(const OpParams       &P,
+                const DevBasis<T>    &B,
+                const FluxFactors<T> &F,
+                int64_t               cell,
+                int                   p,
+                const T (&uplus)[2 * dim],
+                const T (&dplus)[2 * dim],
+                const T (&fan)[2 * dim],
+                const T (&uq)[n],
+                T (&g)[n],
+                const T (&sk)[n],
+                T wd,
+                T (&acc)[n])
+  {
+    constexpr int      h   = n / 2;
+    constexpr bool     odd = n % 2 == 1;
+    const EoLine<n, T> u(uq);
+    // values at the line's two ends
+    T ve = odd ? B.lm * u.m : B.le[0] * u.e[0], vo = B.lo[0] * u.o[0];
 #pragma unroll
-    for (int i = 0; i < n; ++i)
+    for (int i = odd ? 0 : 1; i < h; ++i)
+      ve = fma(B.le[i], u.e[i], ve);
+#pragma unroll
+    for (int i = 1; i < h; ++i)
+      vo = fma(B.lo[i], u.o[i], vo);
+    const T um[2] = {ve + vo, ve - vo};
+    T       f[2], fd[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
       {
-        int q[3];
-        Lay<dim, n>::template idx<dir>(p, i, q);
-        T w = (T)(Bd->w[q[0]] * Bd->w[q[1]]);
-        if (dim == 3)
-          w *= (T)Bd->w[q[2]];
-        g[i] = c0 * w * du[i];
+        const int fc = 2 * dir + s;
+        T         up = uplus[fc];
+        if (!local && !diff && P.has_boundary)
+          {
+            // Dirichlet data, evaluated before the launch
+            // (boundary_value_kernel)
+            const int bi = P.bnd_index[cell * 2 * dim + fc];
+            const T   bv =
+              (T)P.bnd_value[(int64_t)(bi >= 0 ? bi : 0) * Lay<dim, n>::nl +
+                             p];
+            up = bi >= 0 ? bv : up;
+          }
+        const T an = fan[fc], j = um[s] - up;
+        f[s] = fma(an, fma(F.c_own, um[s], F.c_nb * up),
+                   F.c_abs * fabs(an) * j);
+        fd[s] = j;
       }
-    eo_apply<n, true, true, true>(B.eo_D, g, acc);
+    EoSum<n, T> du;
+    if constexpr (skew || diff)
+      eo_derivative<n, false>(B.eo_D, u, du);
+    if constexpr (diff)
+      {
+        // reference derivatives at the two ends
+        T de = odd ? B.dm * u.m : B.de[0] * u.e[0], d_o = B.dd[0] * u.o[0];
+#pragma unroll
+        for (int i = odd ? 0 : 1; i < h; ++i)
+          de = fma(B.de[i], u.e[i], de);
+#pragma unroll
+        for (int i = 1; i < h; ++i)
+          d_o = fma(B.dd[i], u.o[i], d_o);
+        const T dm[2] = {de + d_o, d_o - de};
+        double  vol   = P.h[0] * P.h[1];
+        if (dim == 3)
+          vol *= P.h[2];
+        const double ih = P.inv_h[dir];
+        // W = sign nu/2 times the face weight
+        const T W  = wd * (T)(0.5 * P.sign * P.viscosity * vol * ih);
+        const T si = (T)(P.penalty * ih), tih = (T)ih;
+        const T cd = (T)2 * tih * W;
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+          {
+            const T gs = s ? tih : -tih;
+            const T j  = fd[s];
+            f[s] = fma(W, fma(si, j, -gs * (dm[s] + dplus[2 * dir + s])),
+                       f[s]);
+            fd[s] = -gs * W * j;
+          }
+        // cell diffusion flux sign nu |K| / h^2 w D u
+#pragma unroll
+        for (int i = 0; i < h; ++i)
+          {
+            g[i] = fma(cd * B.w[i], du.e[i] + du.o[i], g[i]);
+            g[n - 1 - i] =
+              fma(cd * B.w[n - 1 - i], du.e[i] - du.o[i], g[n - 1 - i]);
+          }
+        if constexpr (odd)
+          g[h] = fma(cd * B.w[h], du.m, g[h]);
+      }
+    const EoLine<n, T> ge(g);
+    EoSum<n, T>        r;
+    eo_derivative<n, true>(B.eo_D, ge, r);
+    const T fs = f[0] + f[1], fm = f[0] - f[1];
+    const T ds = fd[0] + fd[1], dd = fd[0] - fd[1];
+#pragma unroll
+    for (int q = 0; q < h; ++q)
+      {
+        T se = fma(B.le[q], fs, r.e[q]), so = fma(B.lo[q], fm, r.o[q]);
+        if constexpr (diff)
+          {
+            se = fma(B.de[q], dd, se);
+            so = fma(B.dd[q], ds, so);
+          }
+        acc[q]         = add ? acc[q] + (se + so) : se + so;
+        acc[n - 1 - q] = add ? acc[n - 1 - q] + (se - so) : se - so;
+      }
+    if constexpr (odd)
+      {
+        T sm = fma(B.lm, fs, r.m);
+        if constexpr (diff)
+          sm = fma(B.dm, dd, sm);
+        acc[h] = add ? acc[h] + sm : sm;
+      }
+    if constexpr (skew)
+      {
+#pragma unroll
+        for (int q = 0; q < h; ++q)
+          {
+            acc[q] = fma(sk[q], du.e[q] + du.o[q], acc[q]);
+            acc[n - 1 - q] =
+              fma(sk[n - 1 - q], du.e[q] - du.o[q], acc[n - 1 - q]);
+          }
+        if constexpr (odd)
+          acc[h] = fma(sk[h], du.m, acc[h]);
+      }
   }
 
   // ---- the kernel ------------------------------------------------------------
@@ -575,7 +704,7 @@ namespace dgops
     __shared__ T      s_g1[(AN && dim == 3) ? CPB * STR : 1];
     __shared__ T      s_sk0[(AN && skew) ? CPB * STR : 1];
     __shared__ T      s_sk1[(AN && skew && dim == 3) ? CPB * STR : 1];
-    __shared__ T      s_face[dim == 3 ? CPB * FSTR : 1];
+    __shared__ T      s_face[CPB * FSTR];
     __shared__ T      s_fan[AN ? CPB * 2 * (dim - 1) * nl : 1];
     __shared__ double s_X[CPB * NX];
     // several components (IRK stages): their values at the quadrature
@@ -584,13 +713,12 @@ namespace dgops
     // instead of holding NC lines in registers through the operator phase
     constexpr bool STAGE_LDS = NC > 1;
     __shared__ T   s_stage[STAGE_LDS ? NC * CPB * STR : 1];
-    // several components, 3D advection: the neighbour traces of component
+    // several components, advection: the neighbour traces of component
     // c are interpolated at the start of its operator phase instead of in
     // the value phase, so that one component's traces are live at a time
     // (NC sets of traces held through the operator phase cost one
     // occupancy step)
-    constexpr bool TRACE_LATE =
-      STAGE_LDS && dim == 3 && !diff && fin != fin_local;
+    constexpr bool TRACE_LATE = STAGE_LDS && !diff && fin != fin_local;
     const T *tab_c = static_cast<const T *>(P.tab_cell);
     const T *tab_f = static_cast<const T *>(P.tab_face);
 
@@ -598,9 +726,16 @@ namespace dgops
     const int          tid  = threadIdx.x;
     const int          lc   = tid / nl;
     const int          p    = tid - lc * nl;
-    const int64_t      cell = (int64_t)block * CPB + lc;
-    const bool         active = (lc < CPB) && (cell < P.n_cells);
-    const int          lcs    = lc < CPB ? lc : 0;
+    // threads past the last cell repeat it and store nothing: every load
+    // below is unconditional (a neighbour across a boundary face is read
+    // from the cell itself and replaced by a select). Branches under a
+    // partial exec mask cost moves and split the load batches, and at 250
+    // and more registers the compiler has placed live-range copies before
+    // the mask is restored.
+    const int64_t      cell_t = (int64_t)block * CPB + lc;
+    const bool         active = cell_t < P.n_cells;
+    const int64_t      cell   = active ? cell_t : P.n_cells - 1;
+    const int          lcs    = lc;
 
     T      *u_l   = s_u + lcs * STR;
     T      *acc_l = s_acc + lcs * STR;
@@ -608,7 +743,7 @@ namespace dgops
     T      *g1_l  = (AN && dim == 3) ? s_g1 + lcs * STR : s_g1;
     T      *sk0_l = (AN && skew) ? s_sk0 + lcs * STR : s_sk0;
     T      *sk1_l = (AN && skew && dim == 3) ? s_sk1 + lcs * STR : s_sk1;
-    T      *f_l   = dim == 3 ? s_face + lcs * FSTR : s_face;
+    T      *f_l   = s_face + lcs * FSTR;
     T      *fan_l = AN ? s_fan + lcs * 2 * (dim - 1) * nl : s_fan;
     double *X     = s_X + lcs * NX;
     auto    stage_l = [&](int c) -> T * {
@@ -623,8 +758,7 @@ namespace dgops
     auto          load_own = [&](const T *src, T(&r)[n]) {
 #pragma unroll
       for (int i = 0; i < n; ++i)
-        r[i] =
-          active ? src[cell * nd + L::template off<in_dir>(p, i)] : (T)0;
+        r[i] = src[cell * nd + L::template off<in_dir>(p, i)];
     };
     // waves that are issuing global loads (the cell's values and traces,
     // the tables) or stores get issue priority, so that requests leave
@@ -637,9 +771,8 @@ namespace dgops
     constexpr bool needX = AN || (geo == geo_table && fin != fin_inverse_mass);
     if constexpr (needX)
       {
-        if (active)
-          for (int e = p; e < NX; e += nl)
-            X[e] = P.cell_vertices[cell * NV * dim + e];
+        for (int e = p; e < NX; e += nl)
+          X[e] = P.cell_vertices[cell * NV * dim + e];
       }
     int nb[2 * dim];
     if (dim == 3 && P.morton_bits >= 0)
@@ -654,15 +787,18 @@ namespace dgops
         for (int d = 0; d < dim; ++d)
           {
             const unsigned M = (0x09249249u << d) & full;
-            nb[2 * d] = active ? (int)((((m & M) - 1u) & M) | (m & ~M)) : -1;
-            nb[2 * d + 1] =
-              active ? (int)((((m | ~M) + 1u) & M) | (m & ~M)) : -1;
+            nb[2 * d]     = (int)((((m & M) - 1u) & M) | (m & ~M));
+            nb[2 * d + 1] = (int)((((m | ~M) + 1u) & M) | (m & ~M));
           }
       }
     else
 #pragma unroll
       for (int f = 0; f < 2 * dim; ++f)
-        nb[f] = active ? P.neighbors[cell * 2 * dim + f] : -1;
+        nb[f] = P.neighbors[cell * 2 * dim + f];
+    // the cell a face's neighbour data are read from
+    auto nb_cell = [&](int f) -> int64_t {
+      return nb[f] >= 0 ? (int64_t)nb[f] : cell;
+    };
     if constexpr (needX)
       __syncthreads();
 
@@ -675,38 +811,30 @@ namespace dgops
     T cv[3][n], jxw[n], cvy[n], cvx[n];
     T fan[2 * dim];
     auto load_tables = [&]() {
-        table_line<dim, n>(tab_c, cell, LAST, p, active, cv[LAST]);
+        table_line<dim, n>(tab_c, cell, LAST, p, cv[LAST]);
 #pragma unroll
         for (int d = 0; d < dim; ++d)
           {
-            fan[2 * d] =
-              active ? -tab_f[(cell * dim + d) * nl + p] : (T)0;
-            T up = 0;
-            if (active)
+            fan[2 * d]     = -tab_f[(cell * dim + d) * nl + p];
+            fan[2 * d + 1] = tab_f[(nb_cell(2 * d + 1) * dim + d) * nl + p];
+          }
+        if (P.has_boundary)
+          {
+#pragma unroll
+            for (int f = 0; f < 2 * dim; ++f)
               {
-                const int nbu = nb[2 * d + 1];
-                if (nbu >= 0)
-                  up = tab_f[((int64_t)nbu * dim + d) * nl + p];
-                else
-                  up = (T)P.tab_bnd[((int64_t)P.bnd_index[cell * 2 * dim +
-                                                          2 * d + 1] *
-                                       nl +
-                                     p) *
-                                    (1 + dim)];
+                const int bi = P.bnd_index[cell * 2 * dim + f];
+                const T   an =
+                  (T)P.tab_bnd[((int64_t)(bi >= 0 ? bi : 0) * nl + p) *
+                               (1 + dim)];
+                fan[f] = bi >= 0 ? an : fan[f];
               }
-            fan[2 * d + 1] = up;
-            if (active && nb[2 * d] < 0)
-              fan[2 * d] =
-                (T)P.tab_bnd[((int64_t)P.bnd_index[cell * 2 * dim + 2 * d] *
-                                nl +
-                              p) *
-                             (1 + dim)];
           }
     };
     auto load_speed_rows = [&]() {
       if constexpr (dim == 3)
-        table_line<dim, n>(tab_c, cell, 1, p, active, cvy);
-      table_line<dim, n>(tab_c, cell, 0, p, active, cvx);
+        table_line<dim, n>(tab_c, cell, 1, p, cvy);
+      table_line<dim, n>(tab_c, cell, 0, p, cvx);
     };
 
     // ---- per component: neighbour traces and values at quadrature points
@@ -753,206 +881,110 @@ namespace dgops
             continue;
           }
         // neighbours' face nodes for LDS staging (thread (i, j) loads node
-        // (t1 = i, t2 = j) of every face, one load per face); stored after
-        // the x sweep so that the sweep does not wait for them
-        T tv[6];
-        if constexpr (dim == 3 && !diff && !TRACE_LATE)
+        // (t1 = i, t2 = j) of every face, one load per face; with diffusion
+        // also the nodal derivative normal to the face, from the n values
+        // of the neighbour's line through that node: n loads and n products
+        // per face and thread, where forming it inside the tangential
+        // interpolation takes n^2 of both); stored after the x sweep so
+        // that the sweep does not wait for them
+        constexpr int NTR = diff ? 2 : 1; // trace kinds per face
+        T             tv[NTR][2 * dim];
+        if constexpr (!TRACE_LATE)
           {
-            const int i0 = p % n, j0 = p / n;
+            const int i0 = p % n, j0 = dim == 3 ? p / n : 0;
 #pragma unroll
-            for (int f = 0; f < 6; ++f)
+            for (int f = 0; f < 2 * dim; ++f)
               {
-                const int d = f / 2, s = f % 2;
-                const int t1 = d == 0 ? 1 : 0, t2 = d == 2 ? 1 : 2;
-                tv[f]        = 0;
-                if (active && nb[f] >= 0)
+                constexpr int n2 = n * n;
+                const int     d = f / 2, s = f % 2;
+                const int     st = d == 0 ? 1 : d == 1 ? n : n2;
+                const int     s1 = d == 0 ? n : 1;
+                const int     s2 = d == 2 ? n : n2;
+                const int     lay = s ? 0 : n - 1;
+                const T      *nsrc = src + nb_cell(f) * nd + i0 * s1 +
+                                (dim == 3 ? j0 * s2 : 0);
+                if constexpr (diff)
                   {
-                    int ijk[3];
-                    ijk[d]  = s ? 0 : n - 1;
-                    ijk[t1] = i0;
-                    ijk[t2] = j0;
-                    tv[f]   = src[(int64_t)nb[f] * nd + ijk[0] + n * ijk[1] +
-                                n * n * ijk[2]];
+                    const T(&dp)[max_n] = s ? B.dphi0 : B.dphi1;
+                    T nv[n], dv = 0;
+#pragma unroll
+                    for (int l = 0; l < n; ++l)
+                      nv[l] = nsrc[l * st];
+#pragma unroll
+                    for (int l = 0; l < n; ++l)
+                      dv = fma(dp[l], nv[l], dv);
+                    tv[0][f] = nv[lay];
+                    tv[1][f] = dv;
                   }
+                else
+                  tv[0][f] = nsrc[lay * st];
               }
           }
         // own values, sweep along x
         __builtin_amdgcn_s_setprio(0);
         eo_apply<n, false, false, false>(B.eo_S, r, t);
         lds_write_line<dim, n, 0>(acc_l, p, t);
-        if constexpr (dim == 3 && !diff)
+        if constexpr (!TRACE_LATE)
           {
-            if constexpr (!TRACE_LATE)
-              {
-                const int i0 = p % n, j0 = p / n;
 #pragma unroll
-                for (int f = 0; f < 6; ++f)
-                  f_l[f * nl + j0 * n + i0] = tv[f];
-              }
-          }
-        else if constexpr (dim == 3)
-          {
-            // step 1: thread (aq, j) interpolates the neighbour's face nodes
-            // along the first tangential direction
-            const int aq = p % n, j = p / n;
+            for (int k = 0; k < NTR; ++k)
 #pragma unroll
-            for (int f = 0; f < 6; ++f)
-              {
-                const int d = f / 2, s = f % 2;
-                const int t1 = d == 0 ? 1 : 0, t2 = d == 2 ? 1 : 2;
-                T         v  = 0;
-                if (active && nb[f] >= 0)
-                  {
-                    const T  *nsrc = src + (int64_t)nb[f] * nd;
-                    const int nn   = s ? 0 : n - 1;
-#pragma unroll
-                    for (int i = 0; i < n; ++i)
-                      {
-                        int ijk[3];
-                        ijk[d]  = nn;
-                        ijk[t1] = i;
-                        ijk[t2] = j;
-                        v = fma(B.S[aq][i],
-                                nsrc[ijk[0] + n * ijk[1] + n * n * ijk[2]], v);
-                      }
-                  }
-                f_l[f * nl + j * n + aq] = v;
-                if constexpr (diff)
-                  {
-                    // reference-space derivative of the neighbour normal
-                    // to the face, at its face (nodal derivative at 1 or 0)
-                    const T(&dp)[max_n] = s ? B.dphi0 : B.dphi1;
-                    T         dv        = 0;
-                    if (active && nb[f] >= 0)
-                      {
-                        const T *nsrc = src + (int64_t)nb[f] * nd;
-#pragma unroll
-                        for (int i = 0; i < n; ++i)
-                          {
-                            T dd = 0;
-#pragma unroll
-                            for (int l = 0; l < n; ++l)
-                              {
-                                int ijk[3];
-                                ijk[d]  = l;
-                                ijk[t1] = i;
-                                ijk[t2] = j;
-                                dd      = fma(dp[l],
-                                         nsrc[ijk[0] + n * ijk[1] +
-                                              n * n * ijk[2]],
-                                         dd);
-                              }
-                            dv = fma(B.S[aq][i], dd, dv);
-                          }
-                      }
-                    f_l[(6 + f) * nl + j * n + aq] = dv;
-                  }
-              }
+              for (int f = 0; f < 2 * dim; ++f)
+                f_l[(k * 2 * dim + f) * nl + p] = tv[k][f];
           }
         __syncthreads();
-        T fv[6];
-        if constexpr (dim == 3 && !diff)
+        if constexpr (!TRACE_LATE)
           {
-            if constexpr (!TRACE_LATE)
-            {
             // first tangential interpolation of the staged nodes: thread
-            // (aq, j); written back after the next barrier
-            const int aq = p % n, j = p / n;
+            // (aq, j); in 3D written back after the next barrier
+            const int aq = p % n, j = dim == 3 ? p / n : 0;
 #pragma unroll
-            for (int f = 0; f < 6; ++f)
-              {
-                T v = 0;
+            for (int k = 0; k < NTR; ++k)
 #pragma unroll
-                for (int i = 0; i < n; ++i)
-                  v = fma(B.S[aq][i], f_l[f * nl + j * n + i], v);
-                fv[f] = v;
-              }
-            }
-          }
-        else if constexpr (dim == 3)
-          {
-            // step 2 of the face interpolation: thread (aq, bq)
-            const int aq = p % n, bq = p / n;
+              for (int f = 0; f < 2 * dim; ++f)
+                {
+                  T v = 0;
 #pragma unroll
-            for (int f = 0; f < 6; ++f)
-              {
-                T v = 0;
-#pragma unroll
-                for (int jj = 0; jj < n; ++jj)
-                  v = fma(B.S[bq][jj], f_l[f * nl + jj * n + aq], v);
-                uplus[c][f] = v;
-                if constexpr (diff)
-                  {
-                    T dv = 0;
-#pragma unroll
-                    for (int jj = 0; jj < n; ++jj)
-                      dv = fma(B.S[bq][jj], f_l[(6 + f) * nl + jj * n + aq],
-                               dv);
-                    dplus[c][f] = dv;
-                  }
-              }
-          }
-        else
-          {
-#pragma unroll
-            for (int f = 0; f < 4; ++f)
-              {
-                const int d = f / 2, s = f % 2;
-                T         v = 0, dv = 0;
-                if (active && nb[f] >= 0)
-                  {
-                    const T  *nsrc = src + (int64_t)nb[f] * nd;
-                    const int nn   = s ? 0 : n - 1;
-                    const T(&dp)[max_n] = s ? B.dphi0 : B.dphi1;
-#pragma unroll
-                    for (int i = 0; i < n; ++i)
-                      {
-                        const int ij0 = d == 0 ? nn : i;
-                        const int ij1 = d == 0 ? i : nn;
-                        v = fma(B.S[p][i], nsrc[ij0 + n * ij1], v);
-                        if constexpr (diff)
-                          {
-                            T dd = 0;
-#pragma unroll
-                            for (int l = 0; l < n; ++l)
-                              dd = fma(dp[l],
-                                       nsrc[d == 0 ? l + n * i : i + n * l],
-                                       dd);
-                            dv = fma(B.S[p][i], dd, dv);
-                          }
-                      }
-                  }
-                uplus[c][f] = v;
-                dplus[c][f] = dv;
-              }
+                  for (int i = 0; i < n; ++i)
+                    v = fma(B.S[aq][i],
+                            f_l[(k * 2 * dim + f) * nl + j * n + i], v);
+                  if constexpr (dim == 3)
+                    tv[k][f] = v;
+                  else
+                    (k ? dplus : uplus)[c][f] = v;
+                }
           }
         lds_read_line<dim, n, 1>(acc_l, p, t);
         eo_apply<n, false, false, false>(B.eo_S, t, r);
         if constexpr (dim == 3)
           {
             __syncthreads();
-            if constexpr (!diff && !TRACE_LATE)
+            if constexpr (!TRACE_LATE)
               {
-                const int aq = p % n, j = p / n;
 #pragma unroll
-                for (int f = 0; f < 6; ++f)
-                  f_l[f * nl + j * n + aq] = fv[f];
+                for (int k = 0; k < NTR; ++k)
+#pragma unroll
+                  for (int f = 0; f < 6; ++f)
+                    f_l[(k * 6 + f) * nl + p] = tv[k][f];
               }
             lds_write_line<dim, n, 1>(acc_l, p, r);
             __syncthreads();
-            if constexpr (!diff && !TRACE_LATE)
+            if constexpr (!TRACE_LATE)
               {
                 // second tangential interpolation: thread (aq, bq)
                 const int aq = p % n, bq = p / n;
 #pragma unroll
-                for (int f = 0; f < 6; ++f)
-                  {
-                    T v = 0;
+                for (int k = 0; k < NTR; ++k)
 #pragma unroll
-                    for (int jj = 0; jj < n; ++jj)
-                      v = fma(B.S[bq][jj], f_l[f * nl + jj * n + aq], v);
-                    uplus[c][f] = v;
-                  }
+                  for (int f = 0; f < 6; ++f)
+                    {
+                      T v = 0;
+#pragma unroll
+                      for (int jj = 0; jj < n; ++jj)
+                        v = fma(B.S[bq][jj],
+                                f_l[(k * 6 + f) * nl + jj * n + aq], v);
+                      (k ? dplus : uplus)[c][f] = v;
+                    }
               }
             lds_read_line<dim, n, 2>(acc_l, p, t);
             eo_apply<n, false, false, false>(B.eo_S, t, r);
@@ -970,12 +1002,12 @@ namespace dgops
     // weights at the line's other coordinates; a . n dA on the faces of
     // that line is -+ wl_d(p) |K| / h_d a_d
     double vol = 0, cdir[3] = {0, 0, 0}, wl[3] = {1, 1, 1};
-    if constexpr (UNI)
+    if constexpr (UNI || diff)
       {
         vol = P.h[0] * P.h[1] * (dim == 3 ? P.h[2] : 1.);
 #pragma unroll
         for (int d = 0; d < dim; ++d)
-          cdir[d] = vol / P.h[d] * P.vel_const[d];
+          cdir[d] = vol * P.inv_h[d] * P.vel_const[d];
         int q[3];
 #pragma unroll
         for (int d = 0; d < dim; ++d)
@@ -1015,7 +1047,7 @@ namespace dgops
         load_tables();
         __builtin_amdgcn_s_setprio(0);
         // JxW of the mass term on this thread's line
-        if (fin != fin_inverse_mass && active && P.has_mass)
+        if (fin != fin_inverse_mass && P.has_mass)
           line_jxw<dim, n, LAST, T, L>(X, Bd->xq, Bd->w, p, jxw);
         else
 #pragma unroll
@@ -1027,22 +1059,11 @@ namespace dgops
       int q[3];
       L::template idx<LAST>(p, 0, q);
       T fl[2] = {0, 0};
-      if (active)
-        line_cell_data<dim, n, LAST, true, T>(P, X, Bd, q, cv, jxw, fl);
-      else
-        {
-#pragma unroll
-          for (int i = 0; i < n; ++i)
-            {
-              cv[0][i] = cv[1][i] = cv[2][i] = 0;
-              jxw[i]                         = 1;
-            }
-        }
+      line_cell_data<dim, n, LAST, true, T>(P, X, Bd, q, cv, jxw, fl);
       fan[2 * LAST]     = fl[0];
       fan[2 * LAST + 1] = fl[1];
       constexpr int ntask = dim == 3 ? 4 * n : 2;
-      if (active)
-        for (int task = p; task < ntask; task += nl)
+      for (int task = p; task < ntask; task += nl)
           {
             const int d = dim == 3 ? task / (2 * n) : 0;
             const int s = dim == 3 ? (task / n) % 2 : task;
@@ -1083,64 +1104,68 @@ namespace dgops
             // (t1 = i0, t2 = j0) of each face, then interpolates along t1
             // (thread (aq = i0, j0)) and along t2 (thread (aq = i0, bq = j0))
             const T  *src = io.src + c * io.comp_stride;
-            const int i0 = p % n, j0 = p / n;
-            T         tv[6];
+            const int i0 = p % n, j0 = dim == 3 ? p / n : 0;
+            T         tv[2 * dim];
             __builtin_amdgcn_s_setprio(3);
 #pragma unroll
-            for (int f = 0; f < 6; ++f)
+            for (int f = 0; f < 2 * dim; ++f)
               {
-                const int d = f / 2, s = f % 2;
-                const int t1 = d == 0 ? 1 : 0, t2 = d == 2 ? 1 : 2;
-                tv[f]        = 0;
-                if (active && nb[f] >= 0)
-                  {
-                    int ijk[3];
-                    ijk[d]  = s ? 0 : n - 1;
-                    ijk[t1] = i0;
-                    ijk[t2] = j0;
-                    tv[f]   = src[(int64_t)nb[f] * nd + ijk[0] + n * ijk[1] +
-                                n * n * ijk[2]];
-                  }
+                constexpr int n2 = n * n;
+                const int     d = f / 2, s = f % 2;
+                const int     st = d == 0 ? 1 : d == 1 ? n : n2;
+                const int     s1 = d == 0 ? n : 1;
+                const int     s2 = d == 2 ? n : n2;
+                tv[f] = src[nb_cell(f) * nd + i0 * s1 +
+                            (dim == 3 ? j0 * s2 : 0) + (s ? 0 : n - 1) * st];
               }
             __builtin_amdgcn_s_setprio(0);
 #pragma unroll
-            for (int f = 0; f < 6; ++f)
-              f_l[f * nl + j0 * n + i0] = tv[f];
+            for (int f = 0; f < 2 * dim; ++f)
+              f_l[f * nl + p] = tv[f];
             __syncthreads();
 #pragma unroll
-            for (int f = 0; f < 6; ++f)
+            for (int f = 0; f < 2 * dim; ++f)
               {
                 T v = 0;
 #pragma unroll
                 for (int i = 0; i < n; ++i)
                   v = fma(B.S[i0][i], f_l[f * nl + j0 * n + i], v);
-                tv[f] = v;
+                (dim == 3 ? tv : uplus[0])[f] = v;
               }
-            __syncthreads();
-#pragma unroll
-            for (int f = 0; f < 6; ++f)
-              f_l[f * nl + j0 * n + i0] = tv[f];
-            __syncthreads();
-#pragma unroll
-            for (int f = 0; f < 6; ++f)
+            if constexpr (dim == 3)
               {
-                T v = 0;
+                __syncthreads();
 #pragma unroll
-                for (int jj = 0; jj < n; ++jj)
-                  v = fma(B.S[j0][jj], f_l[f * nl + jj * n + i0], v);
-                uplus[0][f] = v;
+                for (int f = 0; f < 6; ++f)
+                  f_l[f * nl + p] = tv[f];
+                __syncthreads();
+#pragma unroll
+                for (int f = 0; f < 6; ++f)
+                  {
+                    T v = 0;
+#pragma unroll
+                    for (int jj = 0; jj < n; ++jj)
+                      v = fma(B.S[j0][jj], f_l[f * nl + jj * n + i0], v);
+                    uplus[0][f] = v;
+                  }
               }
           }
         const T vf    = (T)P.vel_factor[c];
         const T fcell = (T)(-(1. - P.skew) * P.sign) * vf;
         const T fs    = (T)(P.skew * P.sign) * vf;
-        T       acc[n];
+        const FluxFactors<T> F(P, P.vel_factor[c]);
+        constexpr bool       LOC = fin == fin_local;
+        constexpr bool       MASS = fin != fin_inverse_mass;
+        const T (&up)[2 * dim] = uplus[NUP > 1 ? c : 0];
+        const T (&dp)[2 * dim] = dplus[NUP > 1 ? c : 0];
+        T acc[n];
         // ---- LAST direction (z in 3D, y in 2D) ----
         {
+          if constexpr (MASS)
 #pragma unroll
-          for (int i = 0; i < n; ++i)
-            acc[i] = 0;
-          if (fin != fin_inverse_mass && P.has_mass)
+            for (int i = 0; i < n; ++i)
+              acc[i] = 0;
+          if (MASS && P.has_mass)
             {
 #pragma unroll
               for (int b = 0; b < NC; ++b)
@@ -1155,25 +1180,17 @@ namespace dgops
             }
           T uc[n];
           get_uq(c, uc);
-          T g[n];
+          T g[n], sk[n];
 #pragma unroll
           for (int i = 0; i < n; ++i)
-            g[i] = fcell * cv[LAST][i] * uc[i];
-          eo_apply<n, true, true, true>(B.eo_D, g, acc);
-          if constexpr (skew)
             {
-              T du[n];
-              eo_apply<n, true, false, false>(B.eo_D, uc, du);
-#pragma unroll
-              for (int i = 0; i < n; ++i)
-                acc[i] = fma(fs * cv[LAST][i], du[i], acc[i]);
+              g[i] = fcell * cv[LAST][i] * uc[i];
+              if constexpr (skew)
+                sk[i] = fs * cv[LAST][i];
             }
-          if constexpr (diff)
-            diffusion_cell_term<dim, n, LAST, T>(P, Bd, B, p, uc, acc);
-          face_terms<dim, n, LAST, T, diff, fin == fin_local>(P, Bd, B, cell, p, active, nb,
-                                            uplus[NUP > 1 ? c : 0],
-                                            dplus[NUP > 1 ? c : 0], uc, acc,
-                                            vf, fan);
+          line_operator<dim, n, LAST, T, skew, diff, LOC, MASS>(
+            P, B, F, cell, p, up, dp, fan, uc, g, sk,
+            (T)wl[LAST], acc);
           if constexpr (early_ij)
             {
               // the 1/JxW row of the inverse mass, requested here (the
@@ -1181,7 +1198,7 @@ namespace dgops
               // and x phases instead of after them; no extra registers at
               // the kernel's peak (3D degree 4: 107 VGPRs either way)
               __builtin_amdgcn_s_setprio(3);
-              table_line<dim, n>(tab_c, cell, dim, p, active, ij_row);
+              table_line<dim, n>(tab_c, cell, dim, p, ij_row);
               __builtin_amdgcn_s_setprio(0);
             }
           lds_write_line<dim, n, LAST>(u_l, p, uc);
@@ -1220,7 +1237,7 @@ namespace dgops
         // ---- y direction in 3D ----
         if constexpr (dim == 3)
           {
-            T        uq[n], g[n];
+            T        uq[n], g[n], sk[n];
             const T(&cvd)[n] = cvy;
             lds_read_line<dim, n, 1>(u_l, p, uq);
             if constexpr (AN)
@@ -1232,34 +1249,24 @@ namespace dgops
                   g[i] = fcell * cvd[i] * uq[i];
               }
             lds_read_line<dim, n, 1>(acc_l, p, acc);
-            eo_apply<n, true, true, true>(B.eo_D, g, acc);
-            if constexpr (skew)
+            if constexpr (skew && AN)
+              lds_read_line<dim, n, 1>(sk1_l, p, sk);
+            else if constexpr (skew)
               {
-                T du[n], sk[n];
-                eo_apply<n, true, false, false>(B.eo_D, uq, du);
-                if constexpr (AN)
-                  lds_read_line<dim, n, 1>(sk1_l, p, sk);
-                else
-#pragma unroll
-                  for (int i = 0; i < n; ++i)
-                    sk[i] = fs * cvd[i];
 #pragma unroll
                 for (int i = 0; i < n; ++i)
-                  acc[i] = fma(sk[i], du[i], acc[i]);
+                  sk[i] = fs * cvd[i];
               }
-            if constexpr (diff)
-              diffusion_cell_term<dim, n, 1, T>(P, Bd, B, p, uq, acc);
-            face_terms<dim, n, 1, T, diff, fin == fin_local>(P, Bd, B, cell, p, active, nb,
-                                           uplus[NUP > 1 ? c : 0],
-                                           dplus[NUP > 1 ? c : 0], uq, acc, vf,
-                                           fan);
+            line_operator<dim, n, 1, T, skew, diff, LOC, true>(
+              P, B, F, cell, p, up, dp, fan, uq, g, sk, (T)wl[1],
+              acc);
             lds_write_line<dim, n, 1>(acc_l, p, acc);
             __syncthreads();
           }
 
         // ---- x direction ----
         {
-          T        uq[n], g[n];
+          T        uq[n], g[n], sk[n];
           const T(&cvd)[n] = cvx;
           lds_read_line<dim, n, 0>(u_l, p, uq);
           if constexpr (AN)
@@ -1271,27 +1278,17 @@ namespace dgops
                 g[i] = fcell * cvd[i] * uq[i];
             }
           lds_read_line<dim, n, 0>(acc_l, p, acc);
-          eo_apply<n, true, true, true>(B.eo_D, g, acc);
-          if constexpr (skew)
+          if constexpr (skew && AN)
+            lds_read_line<dim, n, 0>(sk0_l, p, sk);
+          else if constexpr (skew)
             {
-              T du[n], sk[n];
-              eo_apply<n, true, false, false>(B.eo_D, uq, du);
-              if constexpr (AN)
-                lds_read_line<dim, n, 0>(sk0_l, p, sk);
-              else
-#pragma unroll
-                for (int i = 0; i < n; ++i)
-                  sk[i] = fs * cvd[i];
 #pragma unroll
               for (int i = 0; i < n; ++i)
-                acc[i] = fma(sk[i], du[i], acc[i]);
+                sk[i] = fs * cvd[i];
             }
-          if constexpr (diff)
-            diffusion_cell_term<dim, n, 0, T>(P, Bd, B, p, uq, acc);
-          face_terms<dim, n, 0, T, diff, fin == fin_local>(P, Bd, B, cell, p, active, nb,
-                                         uplus[NUP > 1 ? c : 0],
-                                         dplus[NUP > 1 ? c : 0], uq, acc, vf,
-                                         fan);
+          line_operator<dim, n, 0, T, skew, diff, LOC, true>(
+            P, B, F, cell, p, up, dp, fan, uq, g, sk, (T)wl[0],
+            acc);
         }
         __syncthreads();
         if constexpr (fin == fin_local)
@@ -1400,6 +1397,34 @@ namespace dgops
       }
   }
 
+  // Wavefronts per SIMD the compiler has to leave room for. Left alone its
+  // scheduler hoists the loads of a whole phase (there is no branch to stop
+  // at) and takes one or two occupancy steps more than the values need; the
+  // figures are the steps that cost at most a few spilled registers.
+  template <int dim, int n, int NC, typename T, int geo, bool diff, int fin>
+  constexpr int
+  operator_waves()
+  {
+    constexpr bool f64 = sizeof(T) == 8;
+    if (geo == geo_analytic)
+      return 1;
+    if (diff)
+      return 2;
+    if (NC > 1 && fin == fin_integrate)
+      return dim == 3 ? (f64 ? (n <= 2 ? 3 : 2) :
+                               (n <= 5 ? (geo == geo_table ? 4 : 3) : 2)) :
+                        (f64 ? (n <= 4 ? 3 : 2) : (n <= 5 ? 4 : 3));
+    if (dim == 2)
+      return f64 ? (n <= 6 ? 4 : 3) : (n <= 6 ? 6 : 5);
+    if (fin == fin_inverse_mass)
+      return f64 ? (n <= 5 ? 4 : 2) : (n <= 5 ? 6 : 2);
+    if (fin == fin_integrate)
+      // 3D degree 4: 126-128 VGPRs with at most 8 spilled, instead of
+      // 132-146 at three
+      return n <= 5 ? 4 : 2;
+    return 2;
+  }
+
   // One batch of CPB cells per workgroup: workgroup b of n_blocks covers
   // the cells of block xcd_block(b, n_blocks). (A grid-stride loop over
   // several batches per workgroup was measured and rejected: the loop lets
@@ -1407,12 +1432,9 @@ namespace dgops
   // 149 VGPRs at 3D degree 4, one occupancy step lost.)
   template <int dim, int n, int NC, typename T, int geo, bool skew,
             bool diff, int fin, int epi, int CPB>
-  // the single-stage implicit operator (integrate form, 3D, degree <= 4)
-  // at four wavefronts per SIMD: 126-128 VGPRs with at most 4 spilled,
-  // instead of 132-146 at three
   __global__ void __launch_bounds__(CPB * (dim == 3 ? n * n : n))
   __attribute__((amdgpu_waves_per_eu(
-    dim == 3 && NC == 1 && fin == fin_integrate && !diff && n <= 5 ? 4 : 1)))
+    operator_waves<dim, n, NC, T, geo, diff, fin>())))
   dg_operator_kernel(const OpParams                       P,
                      const DevBasis<T> *__restrict__      Bp,
                      const DevBasis<double> *__restrict__ Bd,
@@ -1439,6 +1461,8 @@ namespace dgops
   template <int dim, int n, int NC, typename T, int geo, bool skew,
             bool diff, int fin, int epi, int CPB>
   __global__ void __launch_bounds__(CPB * (dim == 3 ? n * n : n))
+  __attribute__((amdgpu_waves_per_eu(
+    operator_waves<dim, n, NC, T, geo, diff, fin>())))
   dg_operator_batch_kernel(const BatchItem<T> *__restrict__      items,
                            int                                  n_items,
                            const DevBasis<T> *__restrict__      Bp,

@@ -1,0 +1,72 @@
+"""The operator kernel's line terms (cell and face terms on even and odd
+parts, staged traces and normal derivatives) against the CPU oracle where
+they can go wrong: every degree (odd and even numbers of points), ragged last
+workgroups, boundary faces, several components, the speed per point."""
+import numpy as np
+import pytest
+
+from helpers import Cfg, rel_diff
+
+pytestmark = pytest.mark.gpu
+# round-off of two orders of summation in double precision: the oracle's
+# parity bar
+TOL = 1e-12
+
+
+def _apply(c, seed, t=0.1):
+    import torch
+    from advection_miniapp_amd import AdvectionOperation
+    op, o = AdvectionOperation(c.dg()), c.oracle_handle()
+    u = np.random.default_rng(seed).standard_normal(o.n_dofs)
+    dst = op.initialize_dof_vector()
+    op.apply(torch.as_tensor(u, device="cuda"), dst, t)
+    return dst.cpu().numpy(), o.apply(u, t)
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("degree", range(1, 8))
+@pytest.mark.parametrize("speed", ["constant", "per point"])
+def test_sipg_every_degree_on_ragged_meshes(dim, degree, speed):
+    # 3 x 5 (x 1) cells: no tile shape divides the cell count at any degree
+    # above 1, and in 3D a periodic direction has a single cell (its own
+    # neighbour on both sides)
+    kind = 0 if speed == "constant" else (2 if dim == 2 else 1)
+    c = Cfg(dim=dim, degree=degree, n_coarse=[3, 5, 1], refine=0,
+            hi=[1.0, 1.0, 1.0], velocity_kind=kind,
+            velocity=[0.7, -0.4, 0.3], operator_kind=1, viscosity=0.05,
+            penalty_factor=(degree + 1) ** 2)
+    got, ref = _apply(c, 10 * degree + dim)
+    assert rel_diff(got, ref) < TOL
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("degree", range(1, 8))
+@pytest.mark.parametrize("skew", [0.0, 0.5])
+def test_advection_boundary_faces_on_ragged_meshes(dim, degree, skew):
+    c = Cfg(dim=dim, degree=degree, n_coarse=[3, 5, 1], refine=0,
+            hi=[1.0, 1.0, 1.0], perturbation=0.1, periodic=[0, 1, 0],
+            velocity_kind=2 if dim == 2 else 1, flux_alpha=0.5,
+            factor_skew=skew, solution_kind=2,
+            solution_param=[np.pi, 0.0])
+    got, ref = _apply(c, 20 * degree + dim)
+    assert rel_diff(got, ref) < TOL
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("degree,stages", [(1, 3), (2, 3), (3, 2), (5, 2),
+                                           (6, 3)])
+def test_stage_operator_with_boundary_faces(dim, degree, stages):
+    # boundary faces under the kernels with the most registers (2 and 3
+    # stages: the 4-stage table has 7 digits, the oracle computes its own)
+    import torch
+    from advection_miniapp_amd import AdvectionOperation
+    c = Cfg(dim=dim, degree=degree, n_coarse=[3, 2, 1], refine=0,
+            perturbation=0.1, periodic=[1, 0, 0], factor_skew=0.5,
+            velocity_kind=2, solution_kind=2, solution_param=[np.pi, 0.0],
+            irk_stages=stages)
+    op, o = AdvectionOperation(c.dg()), c.oracle_handle()
+    Z = np.random.default_rng(degree).standard_normal(o.n_dofs * stages)
+    op.set_time(0.2, 0.05)
+    dst = op.initialize_dof_vector(blocks=stages)
+    op.vmult_irk(dst, torch.as_tensor(Z, device="cuda"))
+    assert rel_diff(dst.cpu().numpy(), o.irk_vmult(Z, 0.2, 0.05)) < TOL
