@@ -295,15 +295,19 @@ namespace dgops
                   bool            skew,
                   int             fin,
                   int             epi,
-                  const void     *io,
-                  bool            advection_only)
+                  const void     *io)
   {
-    const int diff =
-      op.cfg.operator_kind == DG_OP_ADVECTION_DIFFUSION && !advection_only;
-    if (diff && !P.cartesian)
-      throw Error(DG_ERR_UNSUPPORTED,
-                  "the fused SIPG operator variants are built for "
-                  "axis-aligned meshes (perturbation 0)");
+    const int diff = op.cfg.operator_kind == DG_OP_ADVECTION_DIFFUSION;
+    if (op.sipg_general())
+      {
+        // SIPG on perturbed cells has a kernel of its own
+        if (fp32)
+          throw Error(DG_ERR_UNSUPPORTED,
+                      "SIPG on perturbed cells is built in FP64 (the FP32 "
+                      "variants need axis-aligned cells)");
+        aux_sipg_general(const_cast<Operator &>(op), P, fin, epi, io);
+        return;
+      }
     // axis-aligned cells with a constant transport speed need no tables
     // (products of 1D weights); SIPG with a variable speed evaluates it per
     // point; everything else reads the precomputed geometry tables
@@ -425,27 +429,15 @@ namespace dgops
 
   // the apply in separate passes (advection_solver.cc:661-691: the loop,
   // then the inverse mass): the operator's integration S^T (...) into dst,
-  // the SIPG diffusion terms on perturbed cells added to it, then the
-  // inverse mass matrix in place. Used when the mass matrix is integrated
-  // by QGaussLobatto(k+1) and the operator by QGauss(k+1) (use_gl_quad_mass
-  // alone; the inverse mass is then diag(1 / JxW) at the nodes, :443-445),
-  // and for SIPG on perturbed cells.
-  bool
-  two_pass_apply(const Operator &op)
-  {
-    return op.gl_mass_only || op.sipg_general();
-  }
-
+  // then the inverse mass matrix in place. Used when the mass matrix is
+  // integrated by QGaussLobatto(k+1) and the operator by QGauss(k+1)
+  // (use_gl_quad_mass alone; the inverse mass is then diag(1 / JxW) at the
+  // nodes, :443-445).
   void
   apply_two_pass(Operator &op, const OpParams &P, const void *src, void *dst)
   {
-    const bool general = op.sipg_general();
     if (op.fp32())
       {
-        require(!general,
-                "SIPG on perturbed cells is built in FP64 (the FP32 "
-                "variants need axis-aligned cells)",
-                DG_ERR_UNSUPPORTED);
         OpBuffers<float> io = {};
         io.src   = (const float *)src;
         io.dst   = (float *)dst;
@@ -458,10 +450,7 @@ namespace dgops
         io.src   = (const double *)src;
         io.dst   = (double *)dst;
         io.scale = 1.;
-        launch_operator(op, P, 1, false, true, fin_integrate, epi_store, &io,
-                        general);
-        if (general)
-          aux_sipg_general(op, P, src, dst, 1.);
+        launch_operator(op, P, 1, false, true, fin_integrate, epi_store, &io);
       }
     aux_inverse_mass(op, op.cfg.precision, dst);
   }
@@ -658,7 +647,7 @@ dg_apply(dg_operator *h, const void *src, void *dst, double t)
             "factor_skew = 0",
             DG_ERR_UNSUPPORTED);
     OpParams P = op->base_params(t, 1);
-    if (two_pass_apply(*op))
+    if (op->gl_mass_only)
       {
         apply_two_pass(*op, P, src, dst);
         return;
@@ -719,7 +708,7 @@ namespace dgops
             "perform_stage: the fused LSRK stage is built in FP64 (create "
             "the operator with precision DG_FP64)",
             DG_ERR_UNSUPPORTED);
-    if (two_pass_apply(op))
+    if (op.gl_mass_only)
       {
         // two passes: k = M^-1 (-L ri_in), then the stage update
         const size_t bytes = sizeof(double) * op.n_dofs;

@@ -401,15 +401,8 @@ namespace dgops
       P.sign     = 1.;
       P.has_mass = (with_mass && dt != 0.) ? 1 : 0;
       P.mass[0][0] = dt != 0. ? 1. / dt : 0.;
-      // SIPG on perturbed cells: the advection variant, then the
-      // general-geometry diffusion terms added (FP64)
-      const bool general = op.sipg_general();
       if (fp32)
         {
-          require(!general,
-                  "SIPG on perturbed cells is built in FP64 (the FP32 "
-                  "variants need axis-aligned cells)",
-                  DG_ERR_UNSUPPORTED);
           OpBuffers<float> io = {};
           io.src   = (const float *)src;
           io.dst   = (float *)dst;
@@ -423,9 +416,7 @@ namespace dgops
           io.dst   = (double *)dst;
           io.scale = scale;
           launch_operator(op, P, 1, false, true, fin_integrate, epi_store,
-                          &io, general);
-          if (general)
-            aux_sipg_general(op, P, src, dst, scale);
+                          &io);
         }
     }
 

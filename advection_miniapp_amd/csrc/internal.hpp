@@ -112,7 +112,7 @@ namespace dgops
     // use_gl_quad_mass without use_gl_quad: the mass matrix is integrated
     // with QGaussLobatto(k+1) (its basis in d_mbasis_*), the operator with
     // QGauss(k+1). The apply then runs in two passes; stages keep their
-    // right-hand side in d_gl_k (also for SIPG on perturbed cells)
+    // right-hand side in d_gl_k
     bool   gl_mass_only = false;
     DevBuf d_mbasis_d, d_mbasis_f, d_gl_k;
     // SIPG on perturbed cells: face geometry of the face above every cell
@@ -186,9 +186,8 @@ namespace dgops
     }
     bool fp32() const { return cfg.precision == DG_FP32; }
     size_t scalar_size() const { return fp32() ? 4 : 8; }
-    // SIPG on perturbed (non-axis-aligned) cells: the advection operator
-    // kernel (without its diffusion terms) plus the general-geometry SIPG
-    // kernel, then the inverse mass
+    // SIPG on perturbed (non-axis-aligned) cells: the general-geometry
+    // SIPG kernel
     bool sipg_general() const
     {
       return cfg.operator_kind == DG_OP_ADVECTION_DIFFUSION &&
@@ -198,8 +197,6 @@ namespace dgops
   };
 
   // kernels launched from host code
-  // advection_only: the advection variant also for an advection-diffusion
-  // operator (its diffusion terms come from aux_sipg_general)
   void launch_operator(const Operator &op,
                        const OpParams &P,
                        int             nc,
@@ -207,8 +204,7 @@ namespace dgops
                        bool            skew,
                        int             fin,
                        int             epi,
-                       const void     *io,
-                       bool            advection_only = false);
+                       const void     *io);
 
   // the tile shape for a launch of variant `base_key` (shape bits 0):
   // forced, default, or tuned on first use per device and mesh size class

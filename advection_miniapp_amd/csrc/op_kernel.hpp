@@ -457,6 +457,77 @@ namespace dgops
       }
   }
 
+  // values of the line v at its two ends
+  template <int n, typename T>
+  __device__ __forceinline__ void
+  line_ends(const DevBasis<T> &B, const EoLine<n, T> &v, T (&um)[2])
+  {
+    constexpr int  h   = n / 2;
+    constexpr bool odd = n % 2 == 1;
+    T ve = odd ? B.lm * v.m : B.le[0] * v.e[0], vo = B.lo[0] * v.o[0];
+#pragma unroll
+    for (int i = odd ? 0 : 1; i < h; ++i)
+      ve = fma(B.le[i], v.e[i], ve);
+#pragma unroll
+    for (int i = 1; i < h; ++i)
+      vo = fma(B.lo[i], v.o[i], vo);
+    um[0] = ve + vo;
+    um[1] = ve - vo;
+  }
+
+  // reference derivatives of the line v at its two ends
+  template <int n, typename T>
+  __device__ __forceinline__ void
+  line_end_derivatives(const DevBasis<T> &B, const EoLine<n, T> &v,
+                       T (&dm)[2])
+  {
+    constexpr int  h   = n / 2;
+    constexpr bool odd = n % 2 == 1;
+    T de = odd ? B.dm * v.m : B.de[0] * v.e[0], d_o = B.dd[0] * v.o[0];
+#pragma unroll
+    for (int i = odd ? 0 : 1; i < h; ++i)
+      de = fma(B.de[i], v.e[i], de);
+#pragma unroll
+    for (int i = 1; i < h; ++i)
+      d_o = fma(B.dd[i], v.o[i], d_o);
+    dm[0] = de + d_o;
+    dm[1] = d_o - de;
+  }
+
+  // acc (+)= D^T g + sum_s l_s f[s] (+ sum_s l_s' fd[s] with `diff`)
+  template <int n, bool diff, bool add, typename T>
+  __device__ __forceinline__ void
+  line_integrate(const DevBasis<T> &B, const T (&g)[n], T f0, T f1, T fd0,
+                 T fd1, T (&acc)[n])
+  {
+    constexpr int      h   = n / 2;
+    constexpr bool     odd = n % 2 == 1;
+    const EoLine<n, T> ge(g);
+    EoSum<n, T>        r;
+    eo_derivative<n, true>(B.eo_D, ge, r);
+    const T fs = f0 + f1, fm = f0 - f1;
+    const T ds = fd0 + fd1, dd = fd0 - fd1;
+#pragma unroll
+    for (int q = 0; q < h; ++q)
+      {
+        T se = fma(B.le[q], fs, r.e[q]), so = fma(B.lo[q], fm, r.o[q]);
+        if constexpr (diff)
+          {
+            se = fma(B.de[q], dd, se);
+            so = fma(B.dd[q], ds, so);
+          }
+        acc[q]         = add ? acc[q] + (se + so) : se + so;
+        acc[n - 1 - q] = add ? acc[n - 1 - q] + (se - so) : se - so;
+      }
+    if constexpr (odd)
+      {
+        T sm = fma(B.lm, fs, r.m);
+        if constexpr (diff)
+          sm = fma(B.dm, dd, sm);
+        acc[h] = add ? acc[h] + sm : sm;
+      }
+  }
+
   // Per-launch factors of one component's terms, uniform over the grid:
   // flux = an (c_own u- + c_nb u+) + c_abs |an| (u- - u+) is sign times the
   // numerical flux 1/2 [(u- + u+) an + alpha |an| (u- - u+)] - skew an u-
@@ -520,15 +591,8 @@ namespace dgops
     constexpr int      h   = n / 2;
     constexpr bool     odd = n % 2 == 1;
     const EoLine<n, T> u(uq);
-    // values at the line's two ends
-    T ve = odd ? B.lm * u.m : B.le[0] * u.e[0], vo = B.lo[0] * u.o[0];
-#pragma unroll
-    for (int i = odd ? 0 : 1; i < h; ++i)
-      ve = fma(B.le[i], u.e[i], ve);
-#pragma unroll
-    for (int i = 1; i < h; ++i)
-      vo = fma(B.lo[i], u.o[i], vo);
-    const T um[2] = {ve + vo, ve - vo};
+    T um[2];
+    line_ends<n>(B, u, um);
     T       f[2], fd[2];
 #pragma unroll
     for (int s = 0; s < 2; ++s)
@@ -555,15 +619,8 @@ namespace dgops
       eo_derivative<n, false>(B.eo_D, u, du);
     if constexpr (diff)
       {
-        // reference derivatives at the two ends
-        T de = odd ? B.dm * u.m : B.de[0] * u.e[0], d_o = B.dd[0] * u.o[0];
-#pragma unroll
-        for (int i = odd ? 0 : 1; i < h; ++i)
-          de = fma(B.de[i], u.e[i], de);
-#pragma unroll
-        for (int i = 1; i < h; ++i)
-          d_o = fma(B.dd[i], u.o[i], d_o);
-        const T dm[2] = {de + d_o, d_o - de};
+        T dm[2];
+        line_end_derivatives<n>(B, u, dm);
         double  vol   = P.h[0] * P.h[1];
         if (dim == 3)
           vol *= P.h[2];
@@ -592,30 +649,7 @@ namespace dgops
         if constexpr (odd)
           g[h] = fma(cd * B.w[h], du.m, g[h]);
       }
-    const EoLine<n, T> ge(g);
-    EoSum<n, T>        r;
-    eo_derivative<n, true>(B.eo_D, ge, r);
-    const T fs = f[0] + f[1], fm = f[0] - f[1];
-    const T ds = fd[0] + fd[1], dd = fd[0] - fd[1];
-#pragma unroll
-    for (int q = 0; q < h; ++q)
-      {
-        T se = fma(B.le[q], fs, r.e[q]), so = fma(B.lo[q], fm, r.o[q]);
-        if constexpr (diff)
-          {
-            se = fma(B.de[q], dd, se);
-            so = fma(B.dd[q], ds, so);
-          }
-        acc[q]         = add ? acc[q] + (se + so) : se + so;
-        acc[n - 1 - q] = add ? acc[n - 1 - q] + (se - so) : se - so;
-      }
-    if constexpr (odd)
-      {
-        T sm = fma(B.lm, fs, r.m);
-        if constexpr (diff)
-          sm = fma(B.dm, dd, sm);
-        acc[h] = add ? acc[h] + sm : sm;
-      }
+    line_integrate<n, diff, add>(B, g, f[0], f[1], fd[0], fd[1], acc);
     if constexpr (skew)
       {
 #pragma unroll

@@ -1,18 +1,11 @@
-// SIPG diffusion terms of advection_diffusion_solver.cc:531-613 on cells of
-// any (multilinear) shape, in integrated form: dst += scale * sign * (the
-// diffusion part of the operator tested with every nodal basis function).
-// The advection part comes from the operator kernel in its integrate form
-// (fin_integrate) and the inverse mass from the line kernel, so the apply
-// on such meshes is three launches.
-//
-// CPB cells per workgroup of 256 threads, each cell with its own block of
-// LDS; every phase strides its tasks (a point, face point or node of one of
-// the workgroup's cells) over the threads. The cell's values, its reference
-// gradients at the Gauss points and the integration run as sum-factorized
-// sweeps in LDS; the cell term's geometry (J, adj J, det J) is evaluated
-// point by point from the 2^dim corners, the faces' from a table built once
-// per mesh (sipg_face_table_kernel). Cell term, with the explicit sign convention
-// (sign = -1):
+// Advection-diffusion (SIPG, advection_diffusion_solver.cc:469-613) on cells
+// of any (multilinear) shape: the whole right-hand side (or implicit
+// operator) in one kernel, laid out as the operator kernel (op_kernel.hpp):
+// one line of n points per thread, sweeps in registers, LDS between the
+// directions. The cell term's geometry (J, adj J, det J) is evaluated point
+// by point along the LAST line from the 2^dim corners; the faces' comes from
+// a table built once per mesh (sipg_face_table_kernel). Cell term, with the
+// explicit sign convention (sign = -1):
 //   sign * int grad v . nu grad u = sum_q grad_ref v . (sign nu w_q adj(J)
 //   J^-T grad_ref u).
 // Faces are element-centric: each cell evaluates its own and the
@@ -30,82 +23,19 @@
 #include "dev_basis.hpp"
 #include "dg_common.hpp"
 #include "line_geometry.hpp"
+#include "op_kernel.hpp"
 
 namespace dgops
 {
+  // layout of the face table
   template <int dim, int n>
-  struct SipgLay
+  struct SipgFaces
   {
-    static constexpr int nd = dim == 3 ? n * n * n : n * n;
-    static constexpr int nf = dim == 3 ? n * n : n;
+    static constexpr int nf = dim == 3 ? n * n : n; // points of a face
     static constexpr int nv = 1 << dim;
-    // face table values per face point: J^-1 n of the cell below the face
-    // (dim), of the cell above it (dim), JxW
+    // values per face point: J^-1 n of the cell below the face (dim), of
+    // the cell above it (dim), JxW
     static constexpr int nt = 2 * dim + 1;
-    // stride of the lexicographic node index along direction d
-    __device__ static constexpr int
-    stride(int d)
-    {
-      return d == 0 ? 1 : d == 1 ? n : n * n;
-    }
-    // per-cell LDS block (doubles): own values, the neighbours' values
-    // across the two faces of a direction, six point buffers of the cell
-    // term (in the face passes: the two faces' geometry [face s][nt][nf] as
-    // seen from this cell), the result, the corners, the face partial sums
-    // [face s][own | neighbour][3 nf] and the face coefficients
-    // [face s][4][nf]
-    static constexpr int oU   = 0;
-    static constexpr int oN   = oU + nd;
-    static constexpr int oA   = oN + 2 * nd;
-    static constexpr int oG   = oA;
-    static constexpr int nA   = 6 * nd > 2 * nt * nf ? 6 * nd : 2 * nt * nf;
-    static constexpr int oR   = oA + nA;
-    static constexpr int oX   = oR + nd;
-    static constexpr int oFW  = oX + nv * dim;
-    static constexpr int oFC  = oFW + 12 * nf;
-    static constexpr int size = oFC + 8 * nf;
-    // threads per workgroup and cells per workgroup: one point task per
-    // thread where the cells allow it, at most 48 KB of LDS
-    static constexpr int NT  = 256;
-    static constexpr int cpb_t = nd >= NT ? 1 : NT / nd;
-    static constexpr int cpb_l = 48 * 1024 / (8 * size);
-    static constexpr int CPB   = cpb_l < 1 ? 1 : cpb_t < cpb_l ? cpb_t : cpb_l;
-  };
-
-  // out[p] (+)= sum_i M[r][i] in[p | r -> i] along direction dir, r the
-  // coordinate of p along dir (trans: M[i][r]); optionally a second term
-  // with (M2, in2). in, in2, out: offsets in the cells' LDS blocks
-  template <int dim, int n, int dir, bool trans, bool two>
-  __device__ __forceinline__ void
-  sipg_sweep(double *lds, const double *M, int in, const double *M2, int in2,
-             int out)
-  {
-    using L          = SipgLay<dim, n>;
-    constexpr int st = L::stride(dir);
-    for (int t = threadIdx.x; t < L::CPB * L::nd; t += L::NT)
-      {
-        const int     lc   = t / L::nd, p = t - lc * L::nd;
-        double       *c    = lds + lc * L::size;
-        const int     r    = (p / st) % n;
-        const int     base = p - r * st;
-        double        s    = 0;
-#pragma unroll
-        for (int i = 0; i < n; ++i)
-          {
-            s = fma(trans ? M[i * n + r] : M[r * n + i], c[in + base + i * st],
-                    s);
-            if constexpr (two)
-              s = fma(trans ? M2[i * n + r] : M2[r * n + i],
-                      c[in2 + base + i * st], s);
-          }
-        c[out + p] = s;
-      }
-  }
-
-  template <int d>
-  struct FaceDir
-  {
-    static constexpr int value = d;
   };
 
   // Geometry of the face above each cell in each direction d (its face
@@ -120,7 +50,7 @@ namespace dgops
   sipg_face_entry(const OpParams &P, const DevBasis<double> &B, int64_t cell,
                   int pt, double *__restrict__ T)
   {
-    using L          = SipgLay<dim, n>;
+    using L          = SipgFaces<dim, n>;
     constexpr int nf = L::nf, NV = L::nv;
     constexpr int t1 = d == 0 ? 1 : 0, t2 = d == 2 ? 1 : 2;
     const int     a = pt % n, b = dim == 3 ? pt / n : 0;
@@ -174,7 +104,7 @@ namespace dgops
                          const DevBasis<double> *__restrict__ Bp,
                          double *__restrict__                 T)
   {
-    constexpr int nf = SipgLay<dim, n>::nf;
+    constexpr int nf = SipgFaces<dim, n>::nf;
     const int64_t e  = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (e >= P.n_cells * dim * nf)
       return;
@@ -190,358 +120,485 @@ namespace dgops
       sipg_face_entry<dim, n, 2>(P, *Bp, cell, pt, T);
   }
 
-  template <int dim, int n>
-  __global__ void __launch_bounds__(256)
-  sipg_general_kernel(const OpParams                       P,
-                      const DevBasis<double> *__restrict__ Bp,
-                      const double *__restrict__           faces,
-                      const double *__restrict__           src,
-                      double *__restrict__                 dst,
-                      double                               scale)
+  // The operator on the cells of one workgroup, in the line layout of the
+  // operator kernel (op_kernel.hpp): every thread owns a line of n points.
+  // Phases: values and neighbour traces at the Gauss points; derivatives and
+  // end values of the y and x lines; the fluxes at the points of the LAST
+  // line (all three derivatives meet there) and at the face points; the
+  // integration along x, y and LAST; back to nodal values. Tangential
+  // derivatives at a face come from the traces of all its points (LDS), and
+  // their share of the test functions' normal derivative is integrated over
+  // the face the same way.
+  // Bound by LDS and memory latency at two wavefronts per SIMD: degree 3 in
+  // 3D, 32^3 cells, takes 62 us on one MI355X (three at 168 registers spill
+  // and take 120 us). Before, the advection kernel in integrate form, a
+  // diffusion kernel with one point per task and all operands in LDS, and
+  // the inverse mass took 25 + 129 + 16 us: three passes over the vector,
+  // and 2 to 3 LDS reads per product.
+  template <int dim, int n, bool skew, int fin, int epi>
+  __global__ void __launch_bounds__(block_cells(dim == 3 ? n * n : n) *
+                                    (dim == 3 ? n * n : n))
+  __attribute__((amdgpu_waves_per_eu(2)))
+  sipg_operator_kernel(const OpParams                       P,
+                       const DevBasis<double> *__restrict__ Bp,
+                       const double *__restrict__           faces,
+                       const OpBuffers<double>              io)
   {
-    using L           = SipgLay<dim, n>;
-    constexpr int nd  = L::nd, nf = L::nf, NV = L::nv, NT = L::NT;
-    constexpr int CPB = L::CPB, SZ = L::size;
-    __shared__ double lds[CPB * SZ];
-    __shared__ int    nbr[CPB][2 * dim];
-    // the 1D tables (row stride n): S and G at the Gauss points, and the
-    // nodal-basis derivatives at the two faces
-    __shared__ double tS[n * n], tG[n * n], tD[2][n];
+    using L            = Lay<dim, n>;
+    using FT           = SipgFaces<dim, n>;
+    constexpr int nl   = L::nl, nd = L::nd, STR = L::stride;
+    constexpr int NF   = 2 * dim, NV = 1 << dim, LAST = dim - 1;
+    constexpr int CPB  = cells_per_block<dim, n>();
+    constexpr int XS   = NV * dim | 1; // LDS stride of the corners
+    constexpr int nt   = FT::nt;
+    __shared__ double s_u[CPB * STR];
+    __shared__ double s_gx[CPB * STR];
+    __shared__ double s_gy[dim == 3 ? CPB * STR : 1];
+    __shared__ double s_f[CPB * 2 * NF * nl];
+    __shared__ double s_X[CPB * XS];
+    // rows of S and D that a thread picks by its place in the face: from LDS
+    // (a row stride of n | 1 spreads the banks)
+    constexpr int     RS = n | 1;
+    __shared__ double s_S[n * RS], s_D[n * RS];
 
-    const DevBasis<double> &B     = *Bp;
-    const int64_t           cell0 = (int64_t)blockIdx.x * CPB;
-    const int               tid   = threadIdx.x;
-    const double            nu    = P.viscosity;
-    const double            sg    = P.sign;
-    auto cell_of = [&](int lc) { return cell0 + lc; };
-    auto active  = [&](int lc) { return cell0 + lc < P.n_cells; };
-    auto A       = [](int k) { return L::oA + k * nd; };
+    const DevBasis<double> &B   = *Bp;
+    const double           *src = io.src;
+    const int     tid    = threadIdx.x;
+    const int     lc     = tid / nl;
+    const int     p      = tid - lc * nl;
+    const int64_t cell_t = (int64_t)xcd_block(blockIdx.x, gridDim.x) * CPB + lc;
+    const bool    active = cell_t < P.n_cells;
+    // threads past the last cell repeat it and store nothing
+    const int64_t cell = active ? cell_t : P.n_cells - 1;
+    double       *u_l = s_u + lc * STR, *gx_l = s_gx + lc * STR;
+    double       *gy_l = s_gy + (dim == 3 ? lc * STR : 0);
+    double       *f_l  = s_f + lc * 2 * NF * nl;
+    double       *X    = s_X + lc * XS;
+    const int     ia   = p % n, ib = dim == 3 ? p / n : 0;
 
-    for (int t = tid; t < CPB * nd; t += NT)
+    // ---- values and traces at the Gauss points --------------------------
+    __builtin_amdgcn_s_setprio(3);
+    double r[n], t[n];
+#pragma unroll
+    for (int i = 0; i < n; ++i)
+      r[i] = src[cell * nd + L::template off<0>(p, i)];
+    for (int e = tid; e < n * n; e += CPB * nl)
       {
-        const int lc = t / nd, p = t - lc * nd;
-        double   *c  = lds + lc * SZ;
-        c[L::oU + p] = active(lc) ? src[cell_of(lc) * nd + p] : 0.;
-        c[L::oR + p] = 0;
+        s_S[(e / n) * RS + e % n] = B.S[e / n][e % n];
+        s_D[(e / n) * RS + e % n] = B.D[e / n][e % n];
       }
-    for (int t = tid; t < CPB * NV * dim; t += NT)
+    int64_t nb[NF]; // SIPG meshes are periodic: every neighbour exists
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+      nb[f] = P.neighbors[cell * NF + f];
+    for (int e = p; e < NV * dim; e += nl)
+      X[e] = P.cell_vertices[cell * NV * dim + e];
+    double up[NF], dp[NF];
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
       {
-        const int lc = t / (NV * dim), e = t - lc * NV * dim;
-        lds[lc * SZ + L::oX + e] =
-          active(lc) ? P.cell_vertices[cell_of(lc) * NV * dim + e] : 0.;
+        constexpr int n2 = n * n;
+        const int     d = f / 2, s = f % 2;
+        const int     st = d == 0 ? 1 : d == 1 ? n : n2;
+        const int     s1 = d == 0 ? n : 1, s2 = d == 2 ? n : n2;
+        const double *q = src + nb[f] * nd + ia * s1 + (dim == 3 ? ib * s2 : 0);
+        const double(&dphi)[max_n] = s ? B.dphi0 : B.dphi1;
+        double nv[n], dv = 0;
+#pragma unroll
+        for (int l = 0; l < n; ++l)
+          nv[l] = q[l * st];
+#pragma unroll
+        for (int l = 0; l < n; ++l)
+          dv = fma(dphi[l], nv[l], dv);
+        up[f] = nv[s ? 0 : n - 1];
+        dp[f] = dv;
       }
-    for (int t = tid; t < CPB * 2 * dim; t += NT)
-      {
-        const int lc = t / (2 * dim), f = t - lc * 2 * dim;
-        nbr[lc][f]   = active(lc) ? P.neighbors[cell_of(lc) * 2 * dim + f] : -1;
-      }
-    for (int e = tid; e < n * n; e += NT)
-      {
-        tS[e] = B.S[e / n][e % n];
-        tG[e] = B.G[e / n][e % n];
-      }
-    for (int e = tid; e < 2 * n; e += NT)
-      tD[e / n][e % n] = e < n ? B.dphi0[e] : B.dphi1[e - n];
+    __builtin_amdgcn_s_setprio(0);
+    eo_apply<n, false, false, false>(B.eo_S, r, t);
+    lds_write_line<dim, n, 0>(u_l, p, t);
+    auto put_traces = [&](const double(&a)[NF], const double(&b)[NF]) {
+#pragma unroll
+      for (int f = 0; f < NF; ++f)
+        {
+          f_l[f * nl + p]        = a[f];
+          f_l[(NF + f) * nl + p] = b[f];
+        }
+    };
+    put_traces(up, dp);
     __syncthreads();
-
-    // ---- cell term: reference gradients at the Gauss points ----
-    int gidx[3]; // A() slot of the reference gradient along each direction
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+      {
+        double v = 0, w = 0;
+#pragma unroll
+        for (int i = 0; i < n; ++i)
+          {
+            v = fma(s_S[ia * RS + i], f_l[f * nl + ib * n + i], v);
+            w = fma(s_S[ia * RS + i], f_l[(NF + f) * nl + ib * n + i], w);
+          }
+        up[f] = v;
+        dp[f] = w;
+      }
+    lds_read_line<dim, n, 1>(u_l, p, t);
+    eo_apply<n, false, false, false>(B.eo_S, t, r);
     if constexpr (dim == 3)
       {
-        sipg_sweep<3, n, 0, false, false>(lds, tS, L::oU, tS, L::oU, A(0));
-        sipg_sweep<3, n, 0, false, false>(lds, tG, L::oU, tG, L::oU, A(1));
         __syncthreads();
-        sipg_sweep<3, n, 1, false, false>(lds, tS, A(0), tS, A(0), A(2));
-        sipg_sweep<3, n, 1, false, false>(lds, tS, A(1), tS, A(1), A(3));
-        sipg_sweep<3, n, 1, false, false>(lds, tG, A(0), tG, A(0), A(4));
+        put_traces(up, dp);
+        lds_write_line<dim, n, 1>(u_l, p, r);
         __syncthreads();
-        sipg_sweep<3, n, 2, false, false>(lds, tG, A(2), tG, A(2), A(5));
-        sipg_sweep<3, n, 2, false, false>(lds, tS, A(3), tS, A(3), A(0));
-        sipg_sweep<3, n, 2, false, false>(lds, tS, A(4), tS, A(4), A(1));
-        gidx[0] = 0;
-        gidx[1] = 1;
-        gidx[2] = 5;
-      }
-    else
-      {
-        sipg_sweep<2, n, 0, false, false>(lds, tS, L::oU, tS, L::oU, A(0));
-        sipg_sweep<2, n, 0, false, false>(lds, tG, L::oU, tG, L::oU, A(1));
-        __syncthreads();
-        sipg_sweep<2, n, 1, false, false>(lds, tS, A(1), tS, A(1), A(2));
-        sipg_sweep<2, n, 1, false, false>(lds, tG, A(0), tG, A(0), A(3));
-        gidx[0] = 2;
-        gidx[1] = 3;
-        gidx[2] = 3;
+#pragma unroll
+        for (int f = 0; f < NF; ++f)
+          {
+            double v = 0, w = 0;
+#pragma unroll
+            for (int j = 0; j < n; ++j)
+              {
+                v = fma(s_S[ib * RS + j], f_l[f * nl + j * n + ia], v);
+                w = fma(s_S[ib * RS + j], f_l[(NF + f) * nl + j * n + ia], w);
+              }
+            up[f] = v;
+            dp[f] = w;
+          }
+        lds_read_line<dim, n, 2>(u_l, p, t);
+        eo_apply<n, false, false, false>(B.eo_S, t, r);
       }
     __syncthreads();
-    // point-wise: H_d = sign nu w adj(J)_d . J^-T g (in place of g)
-    for (int t = tid; t < CPB * nd; t += NT)
+
+    // ---- derivatives and end values along every direction ----------------
+    // r: values on the LAST line; dm: own end derivatives; the own and the
+    // neighbours' end values go to LDS (face slots f and NF + f)
+    double           dm[NF];
+    EoSum<n, double> dl; // derivative along the LAST line
+    auto ends = [&](const EoLine<n, double> &v, int d) {
+      double a[2], b[2];
+      line_ends<n>(B, v, a);
+      line_end_derivatives<n>(B, v, b);
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+        {
+          f_l[(2 * d + s) * nl + p] = a[s];
+          dm[2 * d + s]             = b[s];
+        }
+    };
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+      f_l[(NF + f) * nl + p] = up[f];
+    auto expand = [](const EoSum<n, double> &e, double(&o)[n]) {
+      constexpr int h = n / 2;
+#pragma unroll
+      for (int q = 0; q < h; ++q)
+        {
+          o[q]         = e.e[q] + e.o[q];
+          o[n - 1 - q] = e.e[q] - e.o[q];
+        }
+      if constexpr (n % 2 == 1)
+        o[h] = e.m;
+    };
+    lds_write_line<dim, n, LAST>(u_l, p, r);
+    {
+      const EoLine<n, double> v(r);
+      ends(v, LAST);
+      eo_derivative<n, false>(B.eo_D, v, dl);
+    }
+    __syncthreads();
+    {
+      double            q[n];
+      EoSum<n, double> e;
+      lds_read_line<dim, n, 0>(u_l, p, q);
+      const EoLine<n, double> v(q);
+      ends(v, 0);
+      eo_derivative<n, false>(B.eo_D, v, e);
+      expand(e, q);
+      lds_write_line<dim, n, 0>(gx_l, p, q);
+    }
+    if constexpr (dim == 3)
       {
-        const int lc = t / nd, p = t - lc * nd;
-        double   *c  = lds + lc * SZ;
-        const int q[3] = {p % n, (p / n) % n, dim == 3 ? p / (n * n) : 0};
-        double    xi[3] = {B.xq[q[0]], B.xq[q[1]], dim == 3 ? B.xq[q[2]] : 0.};
-        double    x[3], J[3][3], adj[3][3];
-        multilinear_map<dim>(c + L::oX, xi, x, J);
-        const double det = adjugate<dim>(J, adj);
-        double       w   = B.w[q[0]] * B.w[q[1]];
-        if constexpr (dim == 3)
-          w *= B.w[q[2]];
-        double g[3] = {0, 0, 0}, gu[3] = {0, 0, 0};
+        double            q[n];
+        EoSum<n, double> e;
+        lds_read_line<dim, n, 1>(u_l, p, q);
+        const EoLine<n, double> v(q);
+        ends(v, 1);
+        eo_derivative<n, false>(B.eo_D, v, e);
+        expand(e, q);
+        lds_write_line<dim, n, 1>(gy_l, p, q);
+      }
+    __syncthreads();
+
+    // ---- fluxes at the points of the LAST line ---------------------------
+    const double              vf = P.vel_factor[0];
+    const FluxFactors<double> F(P, vf);
+    const double              fcell = -(1. - P.skew) * P.sign * vf;
+    const double              fs    = P.skew * P.sign * vf;
+    double fl[n];  // flux along LAST
+    double acc[n]; // terms tested with the values (mass, skew form)
+    double ij[n];  // 1/JxW
+    {
+      const double *tab = static_cast<const double *>(P.tab_cell);
+      double        g0[n];
+      expand(dl, g0);
+      int q[3];
+      L::template idx<LAST>(p, 0, q);
+      double xi[3] = {B.xq[q[0]], B.xq[q[1]], dim == 3 ? B.xq[q[2]] : 0.};
+      double wl    = B.w[q[0]];
+      double rwl   = B.winv[q[0]];
+      if constexpr (dim == 3)
+        {
+          wl *= B.w[q[1]];
+          rwl *= B.winv[q[1]];
+        }
+      double x[3], J0[3][3], J1[3][3];
+      xi[LAST] = 0.;
+      multilinear_map<dim>(X, xi, x, J0);
+      xi[LAST] = 1.;
+      multilinear_map<dim>(X, xi, x, J1);
+      const double nu = P.sign * P.viscosity;
 #pragma unroll
-        for (int d = 0; d < dim; ++d)
-          g[d] = c[A(gidx[d]) + p];
+      for (int i = 0; i < n; ++i)
+        {
+          // the Jacobian is linear along the line
+          double J[3][3], adj[3][3];
 #pragma unroll
-        for (int e = 0; e < dim; ++e)
+          for (int a = 0; a < dim; ++a)
+#pragma unroll
+            for (int b = 0; b < dim; ++b)
+              J[a][b] = b == LAST ?
+                          J0[a][b] :
+                          fma(B.xq[i], J1[a][b] - J0[a][b], J0[a][b]);
+          const double det = adjugate<dim>(J, adj);
+          // 1/det: hardware estimate and two Newton steps
+          double rd = __builtin_amdgcn_rcp(det);
+          rd        = fma(rd, fma(-det, rd, 1.), rd);
+          rd        = fma(rd, fma(-det, rd, 1.), rd);
+          const double w = wl * B.w[i];
+          ij[i]          = rwl * B.winv[i] * rd;
+          const int    o = L::template off<LAST>(p, i);
+          double       g[3], gu[3], h[3], cv[3];
+          g[LAST] = g0[i];
+          g[0]    = gx_l[o];
+          if constexpr (dim == 3)
+            g[1] = gy_l[o];
+          // diffusion: nu w / det adj(J) adj(J)^T grad_ref u
+#pragma unroll
+          for (int e = 0; e < dim; ++e)
+            {
+              gu[e] = adj[0][e] * g[0];
+#pragma unroll
+              for (int d = 1; d < dim; ++d)
+                gu[e] = fma(adj[d][e], g[d], gu[e]);
+            }
+          const double cd = nu * w * rd;
 #pragma unroll
           for (int d = 0; d < dim; ++d)
-            gu[e] = fma(adj[d][e], g[d], gu[e]);
-        const double f = sg * nu * w / det;
-#pragma unroll
-        for (int d = 0; d < dim; ++d)
-          {
-            double h = 0;
-#pragma unroll
-            for (int e = 0; e < dim; ++e)
-              h = fma(adj[d][e], gu[e], h);
-            c[A(gidx[d]) + p] = f * h;
-          }
-      }
-    __syncthreads();
-    // integration with the test-function gradients
-    if constexpr (dim == 3)
-      {
-        sipg_sweep<3, n, 2, true, false>(lds, tS, A(0), tS, A(0), A(2));
-        sipg_sweep<3, n, 2, true, false>(lds, tS, A(1), tS, A(1), A(3));
-        sipg_sweep<3, n, 2, true, false>(lds, tG, A(5), tG, A(5), A(4));
-        __syncthreads();
-        sipg_sweep<3, n, 1, true, false>(lds, tS, A(2), tS, A(2), A(0));
-        sipg_sweep<3, n, 1, true, true>(lds, tG, A(3), tS, A(4), A(1));
-        __syncthreads();
-        sipg_sweep<3, n, 0, true, true>(lds, tG, A(0), tS, A(1), L::oR);
-      }
-    else
-      {
-        sipg_sweep<2, n, 1, true, false>(lds, tS, A(2), tS, A(2), A(0));
-        sipg_sweep<2, n, 1, true, false>(lds, tG, A(3), tG, A(3), A(1));
-        __syncthreads();
-        sipg_sweep<2, n, 0, true, true>(lds, tG, A(0), tS, A(1), L::oR);
-      }
-    __syncthreads();
-
-    // ---- faces: both faces of a direction per pass (direction d a
-    // compile-time constant, so every index below is static) ----
-    auto face_pair = [&](auto dc) {
-      constexpr int d = decltype(dc)::value;
-      constexpr int t1 = d == 0 ? 1 : 0, t2 = d == 2 ? 1 : 2;
-      constexpr int sd = L::stride(d), s1 = L::stride(t1),
-                    s2 = dim == 3 ? L::stride(t2) : 0;
-      // the neighbours across the two faces (periodic meshes: both exist)
-      for (int t = tid; t < CPB * 2 * nd; t += NT)
-        {
-          const int lc = t / (2 * nd), e = t - lc * 2 * nd;
-          const int s = e / nd, q = e - s * nd;
-          const int nb = nbr[lc][2 * d + s];
-          lds[lc * SZ + L::oN + e] = nb >= 0 ? src[(int64_t)nb * nd + q] : 0.;
-        }
-      // the geometry of the two faces from the table: face 1 is the entry
-      // of this cell, face 0 the entry of the neighbour below, with the two
-      // J^-1 n exchanged and negated (SIPG meshes are periodic: the
-      // neighbour exists)
-      constexpr int nt = L::nt;
-      for (int t = tid; t < CPB * 2 * nf; t += NT)
-        {
-          const int lc = t / (2 * nf), e = t - lc * 2 * nf;
-          const int s = e / nf, pt = e - s * nf;
-          if (!active(lc))
-            continue;
-          const int64_t owner = s ? cell_of(lc) : (int64_t)nbr[lc][2 * d];
-          const double *f     = faces + (owner * dim + d) * nt * nf + pt;
-          double       *g     = lds + lc * SZ + L::oG + s * nt * nf + pt;
-#pragma unroll
-          for (int k = 0; k < dim; ++k)
             {
-              const double own = f[k * nf], other = f[(dim + k) * nf];
-              g[k * nf]         = s ? own : -other;
-              g[(dim + k) * nf] = s ? other : -own;
+              h[d] = adj[d][0] * gu[0];
+#pragma unroll
+              for (int e = 1; e < dim; ++e)
+                h[d] = fma(adj[d][e], gu[e], h[d]);
             }
-          g[2 * dim * nf] = f[2 * dim * nf];
+          // advection: w adj(J) a, from the corners for a constant speed,
+          // else from the geometry table (row d in the order of direction d)
+          if (P.vel_kind == vel_constant)
+            {
+#pragma unroll
+              for (int d = 0; d < dim; ++d)
+                {
+                  double s = adj[d][0] * P.vel_const[0];
+#pragma unroll
+                  for (int e = 1; e < dim; ++e)
+                    s = fma(adj[d][e], P.vel_const[e], s);
+                  cv[d] = w * s;
+                }
+            }
+          else
+            {
+              const double *row = tab + cell * (dim + 1) * nd;
+              if constexpr (dim == 3)
+                {
+                  cv[0] = row[ia * nl + ib + n * i];
+                  cv[1] = row[nd + ib * nl + ia + n * i];
+                }
+              else
+                cv[0] = row[ia * nl + i];
+              cv[LAST] = row[LAST * nd + i * nl + p];
+            }
+          const double uc = r[i];
+          double       v  = 0;
+          if constexpr (fin == fin_integrate)
+            if (P.has_mass)
+              v = P.mass[0][0] * w * det * uc;
+          if constexpr (skew)
+            {
+              double s = cv[0] * g[0];
+#pragma unroll
+              for (int d = 1; d < dim; ++d)
+                s = fma(cv[d], g[d], s);
+              v = fma(fs, s, v);
+            }
+          acc[i]        = v;
+          const double fu = fcell * uc;
+          gx_l[o]       = fma(cd, h[0], fu * cv[0]);
+          if constexpr (dim == 3)
+            gy_l[o] = fma(cd, h[1], fu * cv[1]);
+          fl[i] = fma(cd, h[LAST], fu * cv[LAST]);
+          __builtin_amdgcn_sched_barrier(0);
         }
-      __syncthreads();
-      // layer values and normal derivatives, first tangential direction:
-      // FW[s][side][0..2] = (S v, G v, S dv) at (a, j); side 0 own (layer
-      // s), side 1 the neighbour across face s (its layer 1 - s)
-      for (int t = tid; t < CPB * 4 * nf; t += NT)
+    }
+
+    // ---- fluxes at the face points ---------------------------------------
+    // f, fd: coefficients of the test function and of its reference
+    // derivative normal to the face; c1, c2: of its tangential derivatives
+    double f[NF], fd[NF], c1[NF], c2[NF];
+    {
+      const double *tab_f = static_cast<const double *>(P.tab_face);
+      double        D1[n], D2[n];
+#pragma unroll
+      for (int i = 0; i < n; ++i)
         {
-          const int     lc = t / (4 * nf), e = t - lc * 4 * nf;
-          double       *c  = lds + lc * SZ;
-          const int     s = e / (2 * nf), side = (e / nf) % 2, pt = e % nf;
-          const int     a = pt % n, j = dim == 3 ? pt / n : 0;
-          const double *u  = side ? c + L::oN + s * nd : c + L::oU;
-          const int     ls = side ? 1 - s : s;
-          const int     lay = ls ? n - 1 : 0;
-          const double *dp = tD[ls];
-          double v = 0, vg = 0, dv = 0;
+          D1[i] = s_D[ia * RS + i];
+          if constexpr (dim == 3)
+            D2[i] = s_D[ib * RS + i];
+        }
+#pragma unroll
+      for (int k = 0; k < NF; ++k)
+        {
+          const int d = k / 2, s = k % 2;
+          const int t1 = d == 0 ? 1 : 0, t2 = d == 2 ? 1 : 2;
+          // geometry of this face: face 1 is the entry of this cell, face 0
+          // the entry of the neighbour below, with the two J^-1 n exchanged
+          // and negated
+          const int64_t own = s ? cell : nb[k];
+          const double *T   = faces + (own * dim + d) * nt * nl + p;
+          double        jm[3] = {0, 0, 0}, jp[3] = {0, 0, 0};
+#pragma unroll
+          for (int e = 0; e < dim; ++e)
+            {
+              const double a = T[e * nl], b = T[(dim + e) * nl];
+              jm[e] = s ? a : -b;
+              jp[e] = s ? b : -a;
+            }
+          const double JxW = T[2 * dim * nl];
+          const double an  = s ? tab_f[(nb[k] * dim + d) * nl + p] :
+                                 -tab_f[(cell * dim + d) * nl + p];
+          // tangential derivatives of both traces
+          double g1m = 0, g1p = 0, g2m = 0, g2p = 0;
 #pragma unroll
           for (int i = 0; i < n; ++i)
             {
-              const int    base = i * s1 + j * s2;
-              const double ui   = u[base + lay * sd];
-              double       di   = 0;
-#pragma unroll
-              for (int l = 0; l < n; ++l)
-                di = fma(dp[l], u[base + l * sd], di);
-              v  = fma(tS[a * n + i], ui, v);
-              vg = fma(tG[a * n + i], ui, vg);
-              dv = fma(tS[a * n + i], di, dv);
-            }
-          double *o = c + L::oFW + (2 * s + side) * 3 * nf;
-          o[pt]          = v;
-          o[nf + pt]     = vg;
-          o[2 * nf + pt] = dv;
-        }
-      __syncthreads();
-      // second tangential direction and the flux per face point
-      for (int t = tid; t < CPB * 2 * nf; t += NT)
-        {
-          const int lc = t / (2 * nf), e = t - lc * 2 * nf;
-          double   *c  = lds + lc * SZ;
-          const int s = e / nf, pt = e % nf;
-          const int a = pt % n, b = dim == 3 ? pt / n : 0;
-          double    val[2], gref[2][3];
-#pragma unroll
-          for (int side = 0; side < 2; ++side)
-            {
-              const double *o = c + L::oFW + (2 * s + side) * 3 * nf;
-              double        v = 0, g1 = 0, g2 = 0, gd = 0;
+              g1m = fma(D1[i], f_l[k * nl + ib * n + i], g1m);
+              g1p = fma(D1[i], f_l[(NF + k) * nl + ib * n + i], g1p);
               if constexpr (dim == 3)
                 {
-#pragma unroll
-                  for (int jj = 0; jj < n; ++jj)
-                    {
-                      const int q = jj * n + a;
-                      v  = fma(tS[b * n + jj], o[q], v);
-                      g1 = fma(tS[b * n + jj], o[nf + q], g1);
-                      g2 = fma(tG[b * n + jj], o[q], g2);
-                      gd = fma(tS[b * n + jj], o[2 * nf + q], gd);
-                    }
+                  g2m = fma(D2[i], f_l[k * nl + i * n + ia], g2m);
+                  g2p = fma(D2[i], f_l[(NF + k) * nl + i * n + ia], g2p);
                 }
-              else
-                {
-                  v  = o[a];
-                  g1 = o[nf + a];
-                  gd = o[2 * nf + a];
-                }
-              val[side]      = v;
-              gref[side][d]  = gd;
-              gref[side][t1] = g1;
-              if constexpr (dim == 3)
-                gref[side][t2] = g2;
             }
-          // J^-1 n with this cell's outward normal on both sides, JxW
-          const double *g = c + L::oG + s * nt * nf + pt;
-          double        jn[3] = {0, 0, 0}, jnn[3] = {0, 0, 0};
-#pragma unroll
-          for (int k = 0; k < dim; ++k)
-            {
-              jn[k]  = g[k * nf];
-              jnn[k] = g[(dim + k) * nf];
-            }
-          const double JxW = g[2 * dim * nf];
-          double dnm = 0, dnp = 0;
-#pragma unroll
-          for (int k = 0; k < dim; ++k)
-            {
-              dnm = fma(jn[k], gref[0][k], dnm);
-              dnp = fma(jnn[k], gref[1][k], dnp);
-            }
-          const double sigma   = P.penalty * 0.5 * (fabs(jn[d]) + fabs(jnn[d]));
-          const double jump    = -0.5 * nu * (val[0] - val[1]);
-          const double avg     = -0.5 * nu * (dnm + dnp);
-          const double viscous = jump * sigma - avg;
-          const double cd      = sg * jump * JxW;
-          double      *fc      = c + L::oFC + s * 4 * nf;
-          fc[pt]          = -sg * viscous * JxW;
-          fc[nf + pt]     = cd * jn[d];
-          fc[2 * nf + pt] = cd * jn[t1];
-          fc[3 * nf + pt] = dim == 3 ? cd * jn[t2] : 0.;
+          double dn = fma(jm[d], dm[k], jp[d] * dp[k]);
+          dn        = fma(jm[t1], g1m, fma(jp[t1], g1p, dn));
+          if constexpr (dim == 3)
+            dn = fma(jm[t2], g2m, fma(jp[t2], g2p, dn));
+          const double um = f_l[k * nl + p], un = f_l[(NF + k) * nl + p];
+          const double j  = um - un;
+          const double si = 0.5 * P.penalty * (fabs(jm[d]) + fabs(jp[d]));
+          const double W  = 0.5 * P.sign * P.viscosity * JxW;
+          f[k]            = fma(an, fma(F.c_own, um, F.c_nb * un),
+                     F.c_abs * fabs(an) * j);
+          f[k]            = fma(W, fma(si, j, -dn), f[k]);
+          const double cd = -W * j;
+          fd[k]           = cd * jm[d];
+          c1[k]           = cd * jm[t1];
+          c2[k]           = dim == 3 ? cd * jm[t2] : 0.;
+          // one face's table entries in flight at a time: hoisting those of
+          // all faces costs an occupancy step
+          __builtin_amdgcn_sched_barrier(0);
         }
-      __syncthreads();
-      // test functions: along t2 (transposed) into FW[s][0], then along t1
-      // and onto the nodes; phi_i(s) picks the layer (Gauss-Lobatto nodes),
-      // dphi_s carries the normal-derivative coefficient
-      if constexpr (dim == 3)
+    }
+    __syncthreads();
+    put_traces(c1, c2);
+    __syncthreads();
+    {
+      double D1[n], D2[n];
+#pragma unroll
+      for (int i = 0; i < n; ++i)
         {
-          for (int t = tid; t < CPB * 2 * nf; t += NT)
-            {
-              const int     lc = t / (2 * nf), e = t - lc * 2 * nf;
-              double       *c  = lds + lc * SZ;
-              const int     s = e / nf, pt = e % nf;
-              const int     a = pt % n, i2 = pt / n;
-              const double *fc = c + L::oFC + s * 4 * nf;
-              double        z0 = 0, z1 = 0, z2 = 0, z3 = 0;
-#pragma unroll
-              for (int b = 0; b < n; ++b)
-                {
-                  const int o = b * n + a;
-                  z0 = fma(tS[b * n + i2], fc[o], z0);
-                  z1 = fma(tS[b * n + i2], fc[2 * nf + o], z1);
-                  z2 = fma(tG[b * n + i2], fc[3 * nf + o], z2);
-                  z3 = fma(tS[b * n + i2], fc[nf + o], z3);
-                }
-              double *o = c + L::oFW + 2 * s * 3 * nf;
-              o[pt]          = z0 + z2;
-              o[nf + pt]     = z1;
-              o[2 * nf + pt] = z3;
-            }
-          __syncthreads();
+          D1[i] = s_D[i * RS + ia];
+          if constexpr (dim == 3)
+            D2[i] = s_D[i * RS + ib];
         }
-      for (int t = tid; t < CPB * nd; t += NT)
-        {
-          const int lc = t / nd, p = t - lc * nd;
-          double   *c  = lds + lc * SZ;
-          const int id = (p / sd) % n, i1 = (p / s1) % n;
-          const int i2 = dim == 3 ? (p / s2) % n : 0;
-          double    add = 0;
 #pragma unroll
-          for (int s = 0; s < 2; ++s)
-            {
-              const double *dp = tD[s];
-              const double *o  = c + L::oFW + 2 * s * 3 * nf;
-              const double *fc = c + L::oFC + s * 4 * nf;
-              double        v0 = 0, v1 = 0;
+      for (int k = 0; k < NF; ++k)
 #pragma unroll
-              for (int a = 0; a < n; ++a)
-                {
-                  if constexpr (dim == 3)
-                    {
-                      const int q = i2 * n + a;
-                      v0 = fma(tS[a * n + i1], o[q],
-                               fma(tG[a * n + i1], o[nf + q], v0));
-                      v1 = fma(tS[a * n + i1], o[2 * nf + q], v1);
-                    }
-                  else
-                    {
-                      v0 = fma(tS[a * n + i1], fc[a],
-                               fma(tG[a * n + i1], fc[2 * nf + a], v0));
-                      v1 = fma(tS[a * n + i1], fc[nf + a], v1);
-                    }
-                }
-              add += (id == (s ? n - 1 : 0) ? v0 : 0.) + dp[id] * v1;
-            }
-          c[L::oR + p] += add;
-        }
-      __syncthreads();
-    };
-    face_pair(FaceDir<0>{});
-    face_pair(FaceDir<1>{});
+        for (int i = 0; i < n; ++i)
+          {
+            f[k] = fma(D1[i], f_l[k * nl + ib * n + i], f[k]);
+            if constexpr (dim == 3)
+              f[k] = fma(D2[i], f_l[(NF + k) * nl + i * n + ia], f[k]);
+          }
+    }
+
+    // ---- integration along x, y and LAST ---------------------------------
+    lds_read_line<dim, n, 0>(gx_l, p, t);
+    line_integrate<n, true, false>(B, t, f[0], f[1], fd[0], fd[1], r);
+    lds_write_line<dim, n, 0>(u_l, p, r);
+    __syncthreads();
     if constexpr (dim == 3)
-      face_pair(FaceDir<2>{});
-    for (int t = tid; t < CPB * nd; t += NT)
       {
-        const int lc = t / nd, p = t - lc * nd;
-        if (active(lc))
-          dst[cell_of(lc) * nd + p] += scale * lds[lc * SZ + L::oR + p];
+        lds_read_line<dim, n, 1>(gy_l, p, t);
+        lds_read_line<dim, n, 1>(u_l, p, r);
+        line_integrate<n, true, true>(B, t, f[2], f[3], fd[2], fd[3], r);
+        lds_write_line<dim, n, 1>(u_l, p, r);
+        __syncthreads();
+      }
+    lds_read_line<dim, n, LAST>(u_l, p, r);
+    line_integrate<n, true, true>(B, fl, f[2 * LAST], f[2 * LAST + 1],
+                                  fd[2 * LAST], fd[2 * LAST + 1], r);
+#pragma unroll
+    for (int i = 0; i < n; ++i)
+      {
+        if constexpr (skew || fin == fin_integrate)
+          r[i] += acc[i];
+        if constexpr (fin == fin_inverse_mass)
+          r[i] *= ij[i];
+      }
+
+    // ---- back to nodal values: LAST (registers), x, y --------------------
+    auto back = [&](const double(&a)[n], double(&b)[n]) {
+      if constexpr (fin == fin_inverse_mass)
+        eo_apply<n, false, false, false>(B.eo_Sinv, a, b);
+      else
+        eo_apply<n, false, true, false>(B.eo_S, a, b);
+    };
+    back(r, t);
+    lds_write_line<dim, n, LAST>(u_l, p, t);
+    __syncthreads();
+    lds_read_line<dim, n, 0>(u_l, p, r);
+    back(r, t);
+    constexpr int OUT = dim == 3 ? 1 : 0;
+    if constexpr (dim == 3)
+      {
+        __syncthreads();
+        lds_write_line<dim, n, 0>(u_l, p, t);
+        __syncthreads();
+        lds_read_line<dim, n, 1>(u_l, p, r);
+        back(r, t);
+      }
+    __builtin_amdgcn_s_setprio(3);
+    if (active)
+      {
+#pragma unroll
+        for (int i = 0; i < n; ++i)
+          {
+            const int64_t k = cell * nd + L::template off<OUT>(p, i);
+            if constexpr (epi == epi_store)
+              io.dst[k] = io.scale * t[i];
+            else
+              {
+                const double s0 = io.sol_in[k];
+                io.sol_out[k]   = fma(io.b_dt, t[i], s0);
+                if (!io.last)
+                  io.ri_out[k] = fma(io.a_dt, t[i], s0);
+              }
+          }
       }
   }
 } // namespace dgops

@@ -70,3 +70,38 @@ def test_stage_operator_with_boundary_faces(dim, degree, stages):
     dst = op.initialize_dof_vector(blocks=stages)
     op.vmult_irk(dst, torch.as_tensor(Z, device="cuda"))
     assert rel_diff(dst.cpu().numpy(), o.irk_vmult(Z, 0.2, 0.05)) < TOL
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("degree", range(1, 8))
+@pytest.mark.parametrize("speed", ["constant", "tabulated"])
+def test_sipg_on_perturbed_ragged_meshes(dim, degree, speed):
+    # right-hand side, stage and implicit operator of the general-cell SIPG
+    # kernel; 15 cells fill no workgroup evenly
+    import torch
+    from advection_miniapp_amd import AdvectionOperation
+    kind = 0 if speed == "constant" else (2 if dim == 2 else 1)
+    kw = dict(dim=dim, degree=degree, n_coarse=[3, 5, 2], refine=0, seed=5,
+              perturbation=0.15, velocity_kind=kind, viscosity=0.05,
+              velocity=[0.7, -0.4, 0.3], operator_kind=1,
+              penalty_factor=(degree + 1) ** 2)
+    got, ref = _apply(Cfg(**kw), 30 * degree + dim)
+    assert rel_diff(got, ref) < TOL
+    c = Cfg(factor_skew=0.5, **kw)
+    op, o = AdvectionOperation(c.dg()), c.oracle_handle()
+    u = np.random.default_rng(degree).standard_normal(o.n_dofs)
+    dst = op.initialize_dof_vector()
+    op.set_time(0.2, 0.05)
+    op.vmult(dst, torch.as_tensor(u, device="cuda"))
+    assert rel_diff(dst.cpu().numpy(), o.vmult(u, 0.2, 0.05)) < TOL
+    c = Cfg(**kw)
+    op, o = AdvectionOperation(c.dg()), c.oracle_handle()
+    sol = np.random.default_rng(degree + 50).standard_normal(o.n_dofs)
+    ki, so, nx = np.zeros(o.n_dofs), sol.copy(), np.zeros(o.n_dofs)
+    o.perform_stage(0.1, 0.01, 0.02, u, ki, so, nx)
+    d_sol = torch.as_tensor(sol, device="cuda")
+    d_nx = op.initialize_dof_vector()
+    op.perform_stage(0.1, 0.01, 0.02, torch.as_tensor(u, device="cuda"),
+                     op.initialize_dof_vector(), d_sol, d_nx)
+    assert rel_diff(d_sol.cpu().numpy(), so) < TOL
+    assert rel_diff(d_nx.cpu().numpy(), nx) < TOL
