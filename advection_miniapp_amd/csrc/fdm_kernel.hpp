@@ -91,7 +91,7 @@ namespace dgops
   {
 #pragma unroll
     for (int i = 0; i < n; ++i)
-      v[i] = buf[Lay<dim, n>::template off<dir>(p, mirror<n>(i, rev))];
+      v[i] = buf[Lay<dim, n>::template loff<dir>(p, mirror<n>(i, rev))];
   }
 
   template <int dim, int n, int dir, typename T>
@@ -100,7 +100,7 @@ namespace dgops
   {
 #pragma unroll
     for (int i = 0; i < n; ++i)
-      buf[Lay<dim, n>::template off<dir>(p, mirror<n>(i, rev))] = v[i];
+      buf[Lay<dim, n>::template loff<dir>(p, mirror<n>(i, rev))] = v[i];
   }
 
   // inverse of one block of 2^NB real-pair-coupled points (NB paired
@@ -227,11 +227,12 @@ namespace dgops
             li[0]    = tk.im[0] * m[0];
             nb       = 1;
           }
-        int stride = 1;
 #pragma unroll
         for (int d = 0; d < dim; ++d)
           {
-            const int f = code >> (3 + 4 * d);
+            constexpr int sd[3]  = {1, Lay<dim, n>::sx, Lay<dim, n>::sy};
+            const int     stride = sd[d];
+            const int     f      = code >> (3 + 4 * d);
             base += (f & 7) * stride;
             lr += tk.re[1 + d] * m[1 + d];
             if (f & 8)
@@ -241,7 +242,6 @@ namespace dgops
                 li[nb]    = tk.im[1 + d] * m[1 + d];
                 ++nb;
               }
-            stride *= n;
           }
         fdm_block<NB, Tc>(s_data + lc * NS * STR, base, delta, lr, li,
                           s_cell[lc][3]);

@@ -99,7 +99,9 @@ namespace dgops
                 double (&c)[n])
   {
     const double dth = pi * da;
-    if (fabs(dth) < 0.25)
+    // one choice per wavefront (on axis-aligned cells all lanes agree up to
+    // round-off, and sincospi serves any step): a scalar branch
+    if (__builtin_amdgcn_ballot_w64(!(fabs(dth) < 0.25)) == 0)
       {
         double s0, c0;
         sincospi(a0, &s0, &c0);

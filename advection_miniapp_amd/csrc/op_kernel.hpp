@@ -41,7 +41,41 @@ namespace dgops
   {
     static constexpr int nl = dim == 3 ? n * n : n; // lines per cell
     static constexpr int nd = nl * n;               // dofs per cell
-    static constexpr int stride = nd | 1;           // LDS stride per cell
+
+    // Strides of the y and z coordinates and of the cell in LDS. An even
+    // number of points gets one element of padding per x row: with rows of
+    // 8 (4) values the lanes of a wavefront that read the i-th element of
+    // their x lines share 4 (8) of the 32 double-wide banks, with 9 (5) they
+    // spread over all. Counted over the lanes of a workgroup in all three
+    // directions, the bank cycles per access (1 = no conflict) drop from
+    // 8, 4, 1 to 1, 1, 2 for n = 8 and from 2, 4, 2 to 1, 1, 2 for n = 4
+    // (x, y, z lines, doubles); odd n are conflict free along x already.
+    static constexpr int sx = n % 2 == 1 || (dim == 3 && n == 2) ? n : n + 1;
+    static constexpr int sy = dim == 3 && n == 2 ? 5 : n * sx;
+    static constexpr int stride = dim == 2 ? sy : n == 2 ? 12 : n * sy;
+
+    // LDS offset of point i on line p of direction dir
+    template <int dir>
+    __device__ static __forceinline__ int
+    loff(int p, int i)
+    {
+      if constexpr (dim == 3)
+        {
+          if constexpr (dir == 0)
+            return i + sx * (p % n) + sy * (p / n);
+          else if constexpr (dir == 1)
+            return (p % n) + sx * i + sy * (p / n);
+          else
+            return (p % n) + sx * (p / n) + sy * i;
+        }
+      else
+        {
+          if constexpr (dir == 0)
+            return i + sx * p;
+          else
+            return p + sx * i;
+        }
+    }
 
     // storage offset of point i on line p of direction dir
     template <int dir>
@@ -292,7 +326,7 @@ namespace dgops
   {
 #pragma unroll
     for (int i = 0; i < n; ++i)
-      buf[Lay<dim, n>::template off<dir>(p, i)] = v[i];
+      buf[Lay<dim, n>::template loff<dir>(p, i)] = v[i];
   }
 
   template <int dim, int n, int dir, typename T>
@@ -301,7 +335,7 @@ namespace dgops
   {
 #pragma unroll
     for (int i = 0; i < n; ++i)
-      v[i] = buf[Lay<dim, n>::template off<dir>(p, i)];
+      v[i] = buf[Lay<dim, n>::template loff<dir>(p, i)];
   }
 
   // row `row` of a cell's geometry table [dim + 1][nd] along line p of the
@@ -826,9 +860,15 @@ namespace dgops
           }
       }
     else
+      {
 #pragma unroll
-      for (int f = 0; f < 2 * dim; ++f)
-        nb[f] = P.neighbors[cell * 2 * dim + f];
+        for (int f = 0; f < 2 * dim; ++f)
+          nb[f] = P.neighbors[cell * 2 * dim + f];
+        // wait for them here (vmcnt 0, the others untouched): a wait after
+        // the branches join would hold back the trace loads of the Morton
+        // case behind the cell's own values
+        __builtin_amdgcn_s_waitcnt(0x0F70);
+      }
     // the cell a face's neighbour data are read from
     auto nb_cell = [&](int f) -> int64_t {
       return nb[f] >= 0 ? (int64_t)nb[f] : cell;
@@ -1097,14 +1137,18 @@ namespace dgops
       fan[2 * LAST]     = fl[0];
       fan[2 * LAST + 1] = fl[1];
       constexpr int ntask = dim == 3 ? 4 * n : 2;
-      for (int task = p; task < ntask; task += nl)
-          {
-            const int d = dim == 3 ? task / (2 * n) : 0;
-            const int s = dim == 3 ? (task / n) % 2 : task;
-            const int j = dim == 3 ? task % n : 0;
-            face_line_data<dim, n, LAST, true, T>(
-              P, X, Bd, d, s, j, fan_l + (2 * d + s) * nl + j * n);
-          }
+      // threads without a task of their own repeat the last one (the same
+      // values to the same place) instead of leaving the wavefront
+#pragma unroll 1
+      for (int k = 0; k < (ntask + nl - 1) / nl; ++k)
+        {
+          const int task = min(p + k * nl, ntask - 1);
+          const int d    = dim == 3 ? task / (2 * n) : 0;
+          const int s    = dim == 3 ? (task / n) % 2 : task;
+          const int j    = dim == 3 ? task % n : 0;
+          face_line_data<dim, n, LAST, true, T>(
+            P, X, Bd, d, s, j, fan_l + (2 * d + s) * nl + j * n);
+        }
       __syncthreads();
       const int fidx = dim == 3 ? (p % n) * n + p / n : p;
 #pragma unroll
@@ -1435,7 +1479,8 @@ namespace dgops
   // scheduler hoists the loads of a whole phase (there is no branch to stop
   // at) and takes one or two occupancy steps more than the values need; the
   // figures are the steps that cost at most a few spilled registers.
-  template <int dim, int n, int NC, typename T, int geo, bool diff, int fin>
+  template <int dim, int n, int NC, typename T, int geo, bool skew, bool diff,
+            int fin>
   constexpr int
   operator_waves()
   {
@@ -1451,7 +1496,7 @@ namespace dgops
     if (dim == 2)
       return f64 ? (n <= 6 ? 4 : 3) : (n <= 6 ? 6 : 5);
     if (fin == fin_inverse_mass)
-      return f64 ? (n <= 5 ? 4 : 2) : (n <= 5 ? 6 : 2);
+      return f64 ? (n <= 5 || !skew ? 4 : 2) : (n <= 5 ? 6 : 2);
     if (fin == fin_integrate)
       // 3D degree 4: 126-128 VGPRs with at most 8 spilled, instead of
       // 132-146 at three
@@ -1468,7 +1513,7 @@ namespace dgops
             bool diff, int fin, int epi, int CPB>
   __global__ void __launch_bounds__(CPB * (dim == 3 ? n * n : n))
   __attribute__((amdgpu_waves_per_eu(
-    operator_waves<dim, n, NC, T, geo, diff, fin>())))
+    operator_waves<dim, n, NC, T, geo, skew, diff, fin>())))
   dg_operator_kernel(const OpParams                       P,
                      const DevBasis<T> *__restrict__      Bp,
                      const DevBasis<double> *__restrict__ Bd,
@@ -1496,7 +1541,7 @@ namespace dgops
             bool diff, int fin, int epi, int CPB>
   __global__ void __launch_bounds__(CPB * (dim == 3 ? n * n : n))
   __attribute__((amdgpu_waves_per_eu(
-    operator_waves<dim, n, NC, T, geo, diff, fin>())))
+    operator_waves<dim, n, NC, T, geo, skew, diff, fin>())))
   dg_operator_batch_kernel(const BatchItem<T> *__restrict__      items,
                            int                                  n_items,
                            const DevBasis<T> *__restrict__      Bp,

@@ -372,7 +372,7 @@ namespace dgops
           rd        = fma(rd, fma(-det, rd, 1.), rd);
           const double w = wl * B.w[i];
           ij[i]          = rwl * B.winv[i] * rd;
-          const int    o = L::template off<LAST>(p, i);
+          const int    o = L::template loff<LAST>(p, i);
           double       g[3], gu[3], h[3], cv[3];
           g[LAST] = g0[i];
           g[0]    = gx_l[o];
