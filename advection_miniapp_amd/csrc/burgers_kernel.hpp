@@ -17,8 +17,40 @@ namespace dgops
   // over-integration points per direction: k(k+1)/2 <= 28 at degree 7
   constexpr int max_m = 28;
 
+  // Tables of the line kernel (burgers_line_kernel.hpp): the even-odd form
+  // of an m x n matrix M with M[m-1-q][n-1-i] = M[q][i] (see EvenOdd), and
+  // of the m x m derivative
+  constexpr int burgers_line_max_m = 10;
+
+  struct EvenOddRect
+  {
+    double e[5][2], o[5][2], mc[5], mr[2], mm;
+  };
+  struct EvenOddSquare
+  {
+    double e[5][5], o[5][5], mc[5], mr[5], mm;
+  };
+
+  struct BurgersLineTables
+  {
+    EvenOddRect   S;    // nodal basis at the m points
+    EvenOddRect   R;    // n-point Gauss Lagrange basis at the m points
+    EvenOddSquare eo_D; // collocation derivative of the m points
+    double        le[5], lo[5], lm; // end values, as in DevBasis
+    double        w[burgers_line_max_m], x[burgers_line_max_m];
+  };
+
+  // degrees 2 to 4: the rule determines the test functions (m >= n) and its
+  // tensor fits in LDS
+  constexpr bool
+  burgers_line_degree(int n, int m)
+  {
+    return m >= n && m <= burgers_line_max_m;
+  }
+
   struct BurgersTables
   {
+    BurgersLineTables line;  // where burgers_line_degree()
     int    m;                // over-integration points per direction
     double Sm[max_m][max_n]; // nodal basis at the m Gauss points [q][i]
     double Gm[max_m][max_n]; // its derivative

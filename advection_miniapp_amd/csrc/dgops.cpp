@@ -373,6 +373,68 @@ namespace dgops
       return md;
     }
 
+    // tables of the Burgers line kernel: values of the nodal basis (nodes
+    // xl) and of the n-point Gauss Lagrange basis at the m Gauss points gp,
+    // their collocation derivative and end values, in even-odd form
+    void
+    fill_burgers_line(BurgersLineTables &B, const std::vector<double> &gp,
+                      const std::vector<double>   &gw,
+                      const std::vector<real_ext> &xl, int n)
+    {
+      const int  m  = (int)gp.size();
+      const auto gn = gauss_points_ext(n), gm = gauss_points_ext(m);
+      auto       value = [&](const std::vector<real_ext> &nodes, int i,
+                       real_ext x) {
+        real_ext v, d;
+        lagrange(nodes, i, x, v, d);
+        return (double)v;
+      };
+      auto derivative = [&](int q, int p) {
+        real_ext v, d;
+        lagrange(gm, p, gm[q], v, d);
+        return (double)d;
+      };
+      auto rect = [&](EvenOddRect &E, const std::vector<real_ext> &nodes) {
+        auto M = [&](int q, int i) { return value(nodes, i, gm[q]); };
+        for (int q = 0; q < m / 2; ++q)
+          {
+            for (int i = 0; i < n / 2; ++i)
+              {
+                E.e[q][i] = 0.5 * (M(q, i) + M(q, n - 1 - i));
+                E.o[q][i] = 0.5 * (M(q, i) - M(q, n - 1 - i));
+              }
+            E.mc[q] = M(q, n / 2);
+          }
+        for (int i = 0; i < n / 2; ++i)
+          E.mr[i] = M(m / 2, i);
+        E.mm = M(m / 2, n / 2);
+      };
+      rect(B.S, xl);
+      rect(B.R, gn);
+      for (int q = 0; q < m / 2; ++q)
+        {
+          for (int p = 0; p < m / 2; ++p)
+            {
+              B.eo_D.e[q][p] =
+                0.5 * (derivative(q, p) + derivative(q, m - 1 - p));
+              B.eo_D.o[q][p] =
+                0.5 * (derivative(q, p) - derivative(q, m - 1 - p));
+            }
+          B.eo_D.mc[q] = derivative(q, m / 2);
+          B.eo_D.mr[q] = derivative(m / 2, q);
+          const double a = value(gm, q, 0.0L), b = value(gm, m - 1 - q, 0.0L);
+          B.le[q] = 0.5 * (a + b);
+          B.lo[q] = 0.5 * (a - b);
+        }
+      B.eo_D.mm = derivative(m / 2, m / 2);
+      B.lm      = value(gm, m / 2, 0.0L);
+      for (int q = 0; q < m; ++q)
+        {
+          B.w[q] = gw[q];
+          B.x[q] = gp[q];
+        }
+    }
+
     void
     validate(const dg_config &c)
     {
@@ -547,6 +609,8 @@ dg_create(const dg_config *cfg, void *stream, dg_operator **out)
                 T.Gm[q][i] = (double)dv;
               }
           }
+        if (burgers_line_degree(op->n, m))
+          fill_burgers_line(T.line, gp, gw, xl, op->n);
         op->d_burgers.alloc(sizeof(T));
         hip_check(hipMemcpy(op->d_burgers.ptr, &T, sizeof(T),
                             hipMemcpyHostToDevice),

@@ -92,8 +92,8 @@ FDM_TYPES = {0: ("double", "double", "double"), 1: ("float", "float", "float"),
 
 
 def burgers_variants():
-    # 2D: the point-wise LDS kernel, degrees 1..4; 3D: the slab-wise
-    # kernel, degrees 1..7
+    # degrees 2..4: the line kernel; else 2D: the point-wise LDS kernel
+    # (degree 1), 3D: the slab-wise kernel (degrees 1 and 5..7)
     v = []
     for dim, k, cart, epi in itertools.product((2, 3), range(1, 8), (0, 1),
                                                (EPI_STORE, EPI_LSRK)):
@@ -163,7 +163,8 @@ def emit(path, variants):
             continue
         if var[0] == "burgers":
             _, dim, n, m, cart, epi = var
-            fn = "launch_burgers3" if dim == 3 else "launch_burgers"
+            fn = ("launch_burgers_line" if n <= m <= 10 else
+                  "launch_burgers3" if dim == 3 else "launch_burgers")
             lines.append(
                 f"  static BurgersRegistrar g{i}(burgers_key({dim}, {n}, {cart}, "
                 f"{epi}), &{fn}<{dim}, {n}, {m}, {b(cart)}, {epi}>);")

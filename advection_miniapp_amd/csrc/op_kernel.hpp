@@ -460,9 +460,9 @@ namespace dgops
   // D (transpose: D^T) times the line v; D is skew-centrosymmetric, so the
   // products with v.e are antisymmetric and those with v.o symmetric (see
   // eo_apply, which this equals)
-  template <int n, bool transpose, typename T>
+  template <int n, bool transpose, typename Table, typename T>
   __device__ __forceinline__ void
-  eo_derivative(const EvenOdd<T> &M, const EoLine<n, T> &v, EoSum<n, T> &r)
+  eo_derivative(const Table &M, const EoLine<n, T> &v, EoSum<n, T> &r)
   {
     constexpr int  h   = n / 2;
     constexpr bool odd = n % 2 == 1;
@@ -492,9 +492,9 @@ namespace dgops
   }
 
   // values of the line v at its two ends
-  template <int n, typename T>
+  template <int n, typename Basis, typename T>
   __device__ __forceinline__ void
-  line_ends(const DevBasis<T> &B, const EoLine<n, T> &v, T (&um)[2])
+  line_ends(const Basis &B, const EoLine<n, T> &v, T (&um)[2])
   {
     constexpr int  h   = n / 2;
     constexpr bool odd = n % 2 == 1;
@@ -529,9 +529,9 @@ namespace dgops
   }
 
   // acc (+)= D^T g + sum_s l_s f[s] (+ sum_s l_s' fd[s] with `diff`)
-  template <int n, bool diff, bool add, typename T>
+  template <int n, bool diff, bool add, typename Basis, typename T>
   __device__ __forceinline__ void
-  line_integrate(const DevBasis<T> &B, const T (&g)[n], T f0, T f1, T fd0,
+  line_integrate(const Basis &B, const T (&g)[n], T f0, T f1, T fd0,
                  T fd1, T (&acc)[n])
   {
     constexpr int      h   = n / 2;

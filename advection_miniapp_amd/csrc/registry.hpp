@@ -10,6 +10,7 @@
 
 #include "burgers3d_kernel.hpp"
 #include "burgers_kernel.hpp"
+#include "burgers_line_kernel.hpp"
 #include "colloc_kernel.hpp"
 #include "fdm_kernel.hpp"
 #include "mass_kernel.hpp"
@@ -135,7 +136,30 @@ namespace dgops
     return hipGetLastError();
   }
 
-  // 3D Burgers, degrees 1..7 (slab-wise cell term)
+  // Burgers, degrees 2 to 4 (line kernel)
+  template <int dim, int n, int m, bool cart, int epi>
+  hipError_t
+  launch_burgers_line(const OpParams &P,
+                      const void     *bd,
+                      const void     *tables,
+                      const void     *io,
+                      hipStream_t     stream)
+  {
+    static_assert(burgers_line_degree(n, m), "line kernel degrees");
+    constexpr int CPB    = burgers_line_cells(dim, m);
+    constexpr int T      = CPB * dim * burgers_lines(dim, m);
+    const int64_t blocks = (P.n_cells + CPB - 1) / CPB;
+    if (blocks <= 0)
+      return hipSuccess;
+    hipLaunchKernelGGL((burgers_line_kernel<dim, n, m, cart, epi, CPB>),
+                       dim3((unsigned)blocks), dim3(T), 0, stream, P,
+                       (const DevBasis<double> *)bd,
+                       &((const BurgersTables *)tables)->line,
+                       *(const OpBuffers<double> *)io);
+    return hipGetLastError();
+  }
+
+  // 3D Burgers, degrees 1 and 5..7 (slab-wise cell term)
   template <int dim, int n, int m, bool cart, int epi>
   hipError_t
   launch_burgers3(const OpParams &P,

@@ -69,3 +69,29 @@ def test_burgers_projection_and_lsrk(gpu_lib):
                 ri = sol + ai[s] * dt * k
             sol = new_sol
     assert rel_diff(host(u), sol) < 1e-12
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("pert", [0.0, 0.2])
+def test_burgers_apply_and_stage_on_ragged_meshes(gpu_lib, dim, k, pert):
+    # every kernel of the dispatch (2D point-wise: degree 1; lines: 2 to 4;
+    # slabs: 1 and 5) on boxes of unlike sides whose cells fill no workgroup
+    # evenly, right-hand side and fused stage, with a central-upwind blend
+    if dim == 2 and k > 4:
+        pytest.skip("2D is built for degrees 1..4")
+    c = Cfg(dim=dim, degree=k, n_components=dim, operator_kind=2,
+            n_coarse=[5, 3, 1], refine=0, lo=[-1, 0, 0], hi=[1, 2, 0.5],
+            perturbation=pert, seed=3, flux_alpha=0.7, solution_kind=6)
+    op, o = AdvectionOperation(c.dg()), c.oracle_handle()
+    rng = np.random.default_rng(k + 10 * dim)
+    u, sol = rng.standard_normal((2, o.n_dofs * dim))
+    ref = o.burgers_apply(u)
+    dst = op.initialize_dof_vector()
+    op.apply(dev(u), dst, 0.0)
+    assert rel_diff(host(dst), ref) < 1e-12
+    d_sol, d_nri = dev(sol), op.initialize_dof_vector()
+    op.perform_stage(0.1, 0.01, 0.02, dev(u), op.initialize_dof_vector(),
+                     d_sol, d_nri)
+    assert rel_diff(host(d_sol), sol + 0.01 * ref) < 1e-12
+    assert rel_diff(host(d_nri), sol + 0.02 * ref) < 1e-12
