@@ -23,6 +23,16 @@
 // U = [[1, 1], [i, -i]] (eigenvalues lambda, conj(lambda)) and divides by
 // sigma + sum_d |a_d| lambda_d in complex arithmetic; the same holds for
 // the stage pairs of A^-1. Lines are owned by threads as in op_kernel.hpp.
+//
+// Bound by vector instructions and latency (at degree 4 with three stages
+// the products need 540 fused multiply-adds of a thread; the dofs in and out
+// 39 us at 5 TB/s in FP64). Step 3 works on conjugate halves, reads task
+// records with ready LDS offsets and spreads over both wavefronts, and the
+// sweeps share each table row between the stages: 1410 instead of 2280 vector
+// instructions at degree 4, 2750 instead of 5690 at degree 7, and 126 (FP64)
+// and 72 (FP32) instead of 139 and 109 registers. Degree 4, three stages,
+// 32768 cells on MI355X: FP32 59 -> 43 us, FP64 operator and FDM together
+// 225 -> 206 us.
 #pragma once
 
 #include "op_kernel.hpp"
@@ -33,15 +43,18 @@ namespace dgops
   // direction blocks (n <= 8)
   constexpr int max_fdm_tasks = 128;
 
-  // one step-3 task: a block of real-pair-coupled points of one cell
+  // one step-3 task: a block of real-pair-coupled points of one cell. The
+  // factors are 0 = stage, 1 + d = direction d; the paired ones are listed
+  // first, with the LDS distance of the partner points and the imaginary
+  // part of the eigenvalue.
   template <typename T>
-  struct FdmTask
+  struct alignas(16) FdmTask
   {
-    // bits 0-1: stage block column, bit 2: stage pair; direction d: bits
-    // 3+4d .. 5+4d block column, bit 6+4d pair
-    int code;
-    T   re[4]; // eigenvalue real parts: stage (times 1/dt), directions
-    T   im[4]; // (times |a_d|); imaginary parts, 0 for real blocks
+    int16_t base;      // LDS offset of the first point in the cell's blocks
+    int16_t delta[4];  // of paired factor b
+    uint8_t factor[4]; // of paired factor b
+    T       re[4];     // real parts, factor f times |a_d| or 1/dt
+    T       im[4];     // imaginary parts, of paired factor b
   };
 
   template <typename T>
@@ -77,30 +90,19 @@ namespace dgops
     int64_t       block;         // stage block size (dofs)
   };
 
-  // point i of a line, read or written mirrored when `rev`
-  template <int n>
-  __device__ __forceinline__ int
-  mirror(int i, bool rev)
-  {
-    return rev ? n - 1 - i : i;
-  }
-
-  template <int dim, int n, int dir, typename T>
+  // offsets of the points of LDS line p of direction dir, in reverse order
+  // when `rev`: one start and one step per line
+  template <int dim, int n, int dir>
   __device__ __forceinline__ void
-  lds_read_line_m(const T *buf, int p, bool rev, T (&v)[n])
+  lds_line_m(int p, bool rev, int (&a)[n])
   {
+    using L        = Lay<dim, n>;
+    constexpr int s = dir == 0 ? 1 : dir == 1 ? L::sx : L::sy;
+    const int  step = rev ? -s : s;
+    a[0]            = L::template loff<dir>(p, 0) + (rev ? (n - 1) * s : 0);
 #pragma unroll
-    for (int i = 0; i < n; ++i)
-      v[i] = buf[Lay<dim, n>::template loff<dir>(p, mirror<n>(i, rev))];
-  }
-
-  template <int dim, int n, int dir, typename T>
-  __device__ __forceinline__ void
-  lds_write_line_m(T *buf, int p, bool rev, const T (&v)[n])
-  {
-#pragma unroll
-    for (int i = 0; i < n; ++i)
-      buf[Lay<dim, n>::template loff<dir>(p, mirror<n>(i, rev))] = v[i];
+    for (int i = 1; i < n; ++i)
+      a[i] = a[i - 1] + step;
   }
 
   // inverse of one block of 2^NB real-pair-coupled points (NB paired
@@ -109,142 +111,163 @@ namespace dgops
   // storage distance to the partner along paired factor b, lr the real
   // part of the eigenvalue sum and li[b] the imaginary part of paired
   // factor b (conjugated when the point's bit b is set).
+  //
+  // The values are real, so after U^-1 the point with all bits flipped holds
+  // the conjugate value, before and after the division. Only the 2^(NB-1)
+  // points with bit 0 clear are computed: the transform of bit 0 pairs two
+  // real values to one complex one on the load and splits it on the store.
+  // The factors 1/2 of U^-1 (and 2 of Re, Im at the end) are in `invdet`.
   template <int NB, typename T>
   __device__ __forceinline__ void
   fdm_block(T *data, int base, const int (&delta)[4], T lr,
             const T (&li)[4], T invdet)
   {
-    constexpr int NE = 1 << NB;
-    T             re[NE], im[NE];
-#pragma unroll
-    for (int e = 0; e < NE; ++e)
+    if constexpr (NB == 0)
       {
-        int a = base;
-#pragma unroll
-        for (int b = 0; b < NB; ++b)
-          if ((e >> b) & 1)
-            a += delta[b];
-        re[e] = data[a];
-        im[e] = 0;
+        data[base] *= lr * (invdet / (lr * lr));
+        return;
       }
-    // U^-1 on every pair bit: (x0, x1) -> (1/2 (x0 - i x1), 1/2 (x0 + i x1))
+    // point h: bit b - 1 of h is the bit of paired factor b
+    constexpr int NH = NB == 0 ? 1 : 1 << (NB - 1);
+    int           a[NH];
+    T             re[NH], im[NH];
 #pragma unroll
-    for (int b = 0; b < NB; ++b)
-#pragma unroll
-      for (int e = 0; e < NE; ++e)
-        if (!((e >> b) & 1))
-          {
-            const int e1 = e | (1 << b);
-            const T   r0 = re[e], i0 = im[e], r1 = re[e1], i1 = im[e1];
-            re[e]        = (T)0.5 * (r0 + i1);
-            im[e]        = (T)0.5 * (i0 - r1);
-            re[e1]       = (T)0.5 * (r0 - i1);
-            im[e1]       = (T)0.5 * (i0 + r1);
-          }
-    // times invdet / (lr + i lim_e), lim_e = sum_b +-li[b]: the complement
-    // point (every pair bit flipped) has -lim_e and shares the denominator,
-    // so one division serves both
-    constexpr int NH = NB == 0 ? 1 : NE / 2;
-#pragma unroll
-    for (int e = 0; e < NH; ++e)
+    for (int h = 0; h < NH; ++h)
       {
-        T lim = 0;
+        a[h] = base;
 #pragma unroll
-        for (int b = 0; b < NB; ++b)
-          lim += ((e >> b) & 1) ? -li[b] : li[b];
-        const T q  = invdet / (lr * lr + lim * lim);
+        for (int b = 1; b < NB; ++b)
+          if ((h >> (b - 1)) & 1)
+            a[h] += delta[b];
+        // (x0, x1) -> x0 - i x1
+        re[h] = data[a[h]];
+        im[h] = -data[a[h] + delta[0]];
+      }
+    // U^-1: (z0, z1) -> (z0 - i z1, z0 + i z1)
+#pragma unroll
+    for (int b = 1; b < NB; ++b)
+#pragma unroll
+      for (int h = 0; h < NH; ++h)
+        if (!((h >> (b - 1)) & 1))
+          {
+            const int h1 = h | (1 << (b - 1));
+            const T   r0 = re[h], i0 = im[h], r1 = re[h1], i1 = im[h1];
+            re[h]        = r0 + i1;
+            im[h]        = i0 - r1;
+            re[h1]       = r0 - i1;
+            im[h1]       = i0 + r1;
+          }
+    // times invdet / (lr + i lim_h), lim_h = sum_b +-li[b]
+    const T scale = invdet * (T)(1. / (1 << (NB == 0 ? 0 : NB - 1)));
+#pragma unroll
+    for (int h = 0; h < NH; ++h)
+      {
+        // four divisions at a time (registers for four wavefronts per SIMD instead of three)
+        if constexpr (NB == 4)
+          if (h == 4)
+            asm volatile(""
+                         : "+v"(lr), "+v"(re[0]), "+v"(re[1]), "+v"(re[2]),
+                           "+v"(re[3]));
+        T lim = li[0];
+#pragma unroll
+        for (int b = 1; b < NB; ++b)
+          lim += ((h >> (b - 1)) & 1) ? -li[b] : li[b];
+        const T q  = scale / (lr * lr + lim * lim);
         const T sr = lr * q, si = -lim * q;
-        {
-          const T r = re[e], i = im[e];
-          re[e]     = r * sr - i * si;
-          im[e]     = r * si + i * sr;
-        }
-        if constexpr (NB > 0)
-          {
-            const int ec = e ^ (NE - 1);
-            const T   r  = re[ec], i = im[ec];
-            re[ec]       = r * sr + i * si;
-            im[ec]       = i * sr - r * si;
-          }
+        const T r = re[h], i = im[h];
+        re[h]     = r * sr - i * si;
+        im[h]     = r * si + i * sr;
       }
-    // U on every pair bit: (y+, y-) -> (y+ + y-, i (y+ - y-))
+    // U: (y+, y-) -> (y+ + y-, i (y+ - y-))
 #pragma unroll
-    for (int b = 0; b < NB; ++b)
+    for (int b = 1; b < NB; ++b)
 #pragma unroll
-      for (int e = 0; e < NE; ++e)
-        if (!((e >> b) & 1))
+      for (int h = 0; h < NH; ++h)
+        if (!((h >> (b - 1)) & 1))
           {
-            const int e1 = e | (1 << b);
-            const T   r0 = re[e], i0 = im[e], r1 = re[e1], i1 = im[e1];
-            re[e]        = r0 + r1;
-            im[e]        = i0 + i1;
-            re[e1]       = -(i0 - i1);
-            im[e1]       = r0 - r1;
+            const int h1 = h | (1 << (b - 1));
+            const T   r0 = re[h], i0 = im[h], r1 = re[h1], i1 = im[h1];
+            re[h]        = r0 + r1;
+            im[h]        = i0 + i1;
+            re[h1]       = i1 - i0;
+            im[h1]       = r0 - r1;
           }
+    // y- = conj(y+): (2 Re y+, -2 Im y+)
 #pragma unroll
-    for (int e = 0; e < NE; ++e)
+    for (int h = 0; h < NH; ++h)
       {
-        int a = base;
-#pragma unroll
-        for (int b = 0; b < NB; ++b)
-          if ((e >> b) & 1)
-            a += delta[b];
-        data[a] = re[e];
+        data[a[h]]            = re[h];
+        data[a[h] + delta[0]] = -im[h];
       }
   }
 
   // step 3 for the tasks with NB paired factors of the CPB cells of a
-  // workgroup (task k of cell lc on thread k * CPB + lc, strided by the
-  // workgroup size); s_cell[lc] = (|a_0|, |a_1|, |a_2|, det J^-1)
+  // workgroup (task k of cell lc on thread k * CPB + lc after thread
+  // `first`, strided by the workgroup size); s_cell[lc] = (1/dt,
+  // |a_0|, |a_1|, |a_2|, det J^-1)
   template <int NB, int dim, int n, int NS, int CPB, typename Tc>
   __device__ __forceinline__ void
   fdm_pointwise_group(const FdmDev<Tc> &F, Tc *s_data,
-                      const Tc (*s_cell)[4], int64_t cell0, int64_t n_cells,
-                      Tc idt)
+                      const Tc (*s_cell)[5], int64_t cell0, int64_t n_cells,
+                      int first)
   {
+    const int tid =
+      (int)threadIdx.x - first + ((int)threadIdx.x < first ? blockDim.x : 0);
     constexpr int STR = Lay<dim, n>::stride;
     const int     t0  = F.task_start[NB];
     const int     nt  = (F.task_start[NB + 1] - t0) * CPB;
-    for (int t = threadIdx.x; t < nt; t += blockDim.x)
+    for (int t = tid; t < nt; t += blockDim.x)
       {
         const int k  = t / CPB;
         const int lc = t - k * CPB;
         if (cell0 + lc >= n_cells)
           continue;
-        // one level of independent loads: the task record
-        const FdmTask<Tc> &tk   = F.tasks[t0 + k];
-        const int          code = tk.code;
-        const Tc m[4] = {idt, s_cell[lc][0], s_cell[lc][1], s_cell[lc][2]};
-        // factor 0: stage, 1..dim: directions
-        int base     = (code & 3) * STR;
-        Tc  lr       = tk.re[0] * m[0];
-        int delta[4] = {0, 0, 0, 0};
-        Tc  li[4]    = {0, 0, 0, 0};
-        int nb       = 0;
-        if (code & 4)
-          {
-            delta[0] = STR;
-            li[0]    = tk.im[0] * m[0];
-            nb       = 1;
-          }
+        const FdmTask<Tc> &tk = F.tasks[t0 + k];
+        const Tc          *m  = s_cell[lc];
+        Tc                 lr = tk.re[0] * m[0];
 #pragma unroll
         for (int d = 0; d < dim; ++d)
+          lr += tk.re[1 + d] * m[1 + d];
+        int delta[4];
+        Tc  li[4];
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
           {
-            constexpr int sd[3]  = {1, Lay<dim, n>::sx, Lay<dim, n>::sy};
-            const int     stride = sd[d];
-            const int     f      = code >> (3 + 4 * d);
-            base += (f & 7) * stride;
-            lr += tk.re[1 + d] * m[1 + d];
-            if (f & 8)
-              {
-                // nb < NB <= 4 here
-                delta[nb] = stride;
-                li[nb]    = tk.im[1 + d] * m[1 + d];
-                ++nb;
-              }
+            delta[b] = tk.delta[b];
+            li[b]    = tk.im[b] * m[tk.factor[b]];
           }
-        fdm_block<NB, Tc>(s_data + lc * NS * STR, base, delta, lr, li,
-                          s_cell[lc][3]);
+        fdm_block<NB, Tc>(s_data + lc * NS * STR, tk.base, delta, lr, li,
+                          m[4]);
+      }
+  }
+
+  // A 1D matrix product on the thread's lines of all NS stages, row by row:
+  // out(q, v) gets the values v[j] = sum_i M[q][i] in[j][i] of the stages.
+  // One row of the table is in scalar registers at a time and used for all
+  // stages. The pointer is opaque for every sweep, so that the compiler
+  // loads the rows again (from the scalar cache) instead of keeping a whole
+  // table over the sweeps: n = 8 has 64 doubles, more than there are scalar
+  // registers, and spent 3200 of 6300 vector instructions on spilling them.
+  template <int n, int NS, typename T, typename F>
+  __device__ __forceinline__ void
+  fdm_sweep(const T (&table)[max_n][max_n], const T (&in)[NS][n], F &&out)
+  {
+    using CT = const __attribute__((address_space(4))) T;
+    CT *M    = (CT *)(uintptr_t)&table[0][0];
+    asm volatile("" : "+s"(M));
+#pragma unroll
+    for (int q = 0; q < n; ++q)
+      {
+        T v[NS];
+#pragma unroll
+        for (int j = 0; j < NS; ++j)
+          v[j] = M[q * max_n] * in[j][0];
+#pragma unroll
+        for (int i = 1; i < n; ++i)
+#pragma unroll
+          for (int j = 0; j < NS; ++j)
+            v[j] = fma(M[q * max_n + i], in[j][i], v[j]);
+        out(q, v);
       }
   }
 
@@ -266,151 +289,172 @@ namespace dgops
     const int         tid  = threadIdx.x;
     const int         lc   = tid / nl;
     const int         p    = tid - lc * nl;
-    const int64_t     cell =
-      (int64_t)xcd_block(blockIdx.x, gridDim.x) * CPB + lc;
-    const bool        active = (lc < CPB) && (cell < P.n_cells);
+    const int64_t     cell0 = (int64_t)xcd_block(blockIdx.x, gridDim.x) * CPB;
+    const bool        active = lc < CPB && cell0 + lc < P.n_cells;
     const int         lcs    = lc < CPB ? lc : 0;
     Tc               *data   = s_data + lcs * NS * STR;
+    // idle threads load the last cell and store nothing
+    const int64_t     cell   = cell0 + lcs < P.n_cells ? cell0 + lcs :
+                                                         P.n_cells - 1;
 
-    // |speed| per direction and det J^-1 of the workgroup's cells, read by
-    // any thread in step 3
-    __shared__ Tc s_cell[CPB][4];
+    // 1/dt, |speed| per direction and det J^-1 of the workgroup's cells,
+    // read by any thread in step 3
+    __shared__ Tc s_cell[CPB][5];
     bool rv[3] = {false, false, false};
-    if (active)
+#pragma unroll
+    for (int d = 0; d < dim; ++d)
       {
-        for (int d = 0; d < dim; ++d)
-          {
-            const double a = P.cell_velocity[cell * dim + d] * P.vel_scale;
-            rv[d]          = a < 0.;
-            if (p == 0)
-              s_cell[lc][d] = (Tc)fabs(a);
-          }
-        if (p == 0)
-          s_cell[lc][3] = (Tc)P.cell_invdet[cell];
+        const double a = P.cell_velocity[cell * dim + d] * P.vel_scale;
+        rv[d]          = a < 0.;
+        if (active && p == 0)
+          s_cell[lc][1 + d] = (Tc)fabs(a);
       }
+    if (active && p == 0)
+      {
+        s_cell[lc][0] = (Tc)P.inv_dt;
+        s_cell[lc][4] = (Tc)P.cell_invdet[cell];
+      }
+    // x-line in the vectors, mirrored
+    const int64_t x0 = cell * nd + L::template off<0>(p, 0) +
+                       (rv[0] ? n - 1 : 0);
+    const int     xs = rv[0] ? -1 : 1;
+    Tc            r[NS][n];
+    int           al[n];
 
     // 1-2: load (x mirrored), stage transform, V^-1 M^-1 sweeps x, y, (z)
     // with the y and z mirrors on the LDS reads. Every stage has its own
     // LDS block; a thread rewrites exactly the positions of its own line
     // (the mirrors permute within a line), so all stages share one barrier
     // per direction change.
-    {
-      Tc r[NS][n];
 #pragma unroll
-      for (int t = 0; t < NS; ++t)
+    for (int t = 0; t < NS; ++t)
 #pragma unroll
-        for (int i = 0; i < n; ++i)
-          r[t][i] =
-            active ? (Tc)src[t * P.block + cell * nd +
-                             L::template off<0>(p, mirror<n>(i, rv[0]))] :
-                     (Tc)0;
+      for (int i = 0; i < n; ++i)
+        r[t][i] = (Tc)src[t * P.block + x0 + i * xs];
+    if constexpr (NS > 1)
 #pragma unroll
-      for (int j = 0; j < NS; ++j)
+      for (int i = 0; i < n; ++i)
         {
-          Tc w[n], t[n];
-#pragma unroll
-          for (int i = 0; i < n; ++i)
-            {
-              Tc s = 0;
-#pragma unroll
-              for (int k = 0; k < NS; ++k)
-                s = fma(F.Tinv[j][k], r[k][i], s);
-              w[i] = NS == 1 ? r[0][i] : s;
-            }
-          mat_apply<n>(F.VinvMinv, w, t);
-          lds_write_line<dim, n, 0>(data + j * STR, p, t);
-        }
-      __syncthreads();
-#pragma unroll
-      for (int j = 0; j < NS; ++j)
-        {
-          Tc w[n], t[n];
-          lds_read_line_m<dim, n, 1>(data + j * STR, p, rv[1], t);
-          mat_apply<n>(F.VinvMinv, t, w);
-          lds_write_line<dim, n, 1>(data + j * STR, p, w);
-        }
-      if constexpr (dim == 3)
-        {
-          __syncthreads();
+          Tc w[NS];
 #pragma unroll
           for (int j = 0; j < NS; ++j)
             {
-              Tc w[n], t[n];
-              lds_read_line_m<dim, n, 2>(data + j * STR, p, rv[2], t);
-              mat_apply<n>(F.VinvMinv, t, w);
-              lds_write_line<dim, n, 2>(data + j * STR, p, w);
+              w[j] = 0;
+#pragma unroll
+              for (int k = 0; k < NS; ++k)
+                w[j] = fma(F.Tinv[j][k], r[k][i], w[j]);
             }
+#pragma unroll
+          for (int j = 0; j < NS; ++j)
+            r[j][i] = w[j];
         }
-      __syncthreads();
-    }
+    fdm_sweep<n, NS>(F.VinvMinv, r, [&](int q, const Tc(&v)[NS]) {
+#pragma unroll
+      for (int j = 0; j < NS; ++j)
+        data[j * STR + L::template loff<0>(p, q)] = v[j];
+    });
+    __syncthreads();
+    lds_line_m<dim, n, 1>(p, rv[1], al);
+#pragma unroll
+    for (int j = 0; j < NS; ++j)
+#pragma unroll
+      for (int i = 0; i < n; ++i)
+        r[j][i] = data[j * STR + al[i]];
+    fdm_sweep<n, NS>(F.VinvMinv, r, [&](int q, const Tc(&v)[NS]) {
+#pragma unroll
+      for (int j = 0; j < NS; ++j)
+        data[j * STR + L::template loff<1>(p, q)] = v[j];
+    });
+    if constexpr (dim == 3)
+      {
+        __syncthreads();
+        lds_line_m<dim, n, 2>(p, rv[2], al);
+#pragma unroll
+        for (int j = 0; j < NS; ++j)
+#pragma unroll
+          for (int i = 0; i < n; ++i)
+            r[j][i] = data[j * STR + al[i]];
+        fdm_sweep<n, NS>(F.VinvMinv, r, [&](int q, const Tc(&v)[NS]) {
+#pragma unroll
+          for (int j = 0; j < NS; ++j)
+            data[j * STR + L::template loff<2>(p, q)] = v[j];
+        });
+      }
+    __syncthreads();
 
     // 3: pointwise inverse on the blocks of the workgroup's cells, one
     // group of block shapes (number of paired factors NB) after the other:
-    // the threads of a wave run one shape at a time
+    // the threads of a wave run one shape at a time. The last and costliest
+    // group starts on the second wavefront, the others on the first: with
+    // all of them on the first (five groups of 5 to 100 tasks for n = 5 and
+    // three stages) the second waits for it.
     {
-      const Tc      idt   = (Tc)P.inv_dt;
-      const int64_t cell0 = cell - lc;
+      constexpr int TOP = dim + (NS > 1 ? 1 : 0);
       fdm_pointwise_group<0, dim, n, NS, CPB>(F, s_data, s_cell, cell0,
-                                              P.n_cells, idt);
+                                              P.n_cells, 0);
       fdm_pointwise_group<1, dim, n, NS, CPB>(F, s_data, s_cell, cell0,
-                                              P.n_cells, idt);
+                                              P.n_cells, 0);
       fdm_pointwise_group<2, dim, n, NS, CPB>(F, s_data, s_cell, cell0,
-                                              P.n_cells, idt);
-      if constexpr (dim == 3 || NS > 1)
+                                              P.n_cells, TOP == 2 ? 64 : 0);
+      if constexpr (TOP >= 3)
         fdm_pointwise_group<3, dim, n, NS, CPB>(F, s_data, s_cell, cell0,
-                                                P.n_cells, idt);
-      if constexpr (dim == 3 && NS > 1)
+                                                P.n_cells,
+                                                TOP == 3 ? 64 : 0);
+      if constexpr (TOP >= 4)
         fdm_pointwise_group<4, dim, n, NS, CPB>(F, s_data, s_cell, cell0,
-                                                P.n_cells, idt);
+                                                P.n_cells, 64);
       __syncthreads();
     }
 
+    // the line's offsets again, instead of kept in registers over step 3
+    int pv = p;
+    asm volatile("" : "+v"(pv));
+
     // 4: V sweeps LAST, ..., x with the mirrors on the writes; the x
     // mirror goes into the store
-    Tc w[NS][n];
+    lds_line_m<dim, n, LAST>(pv, rv[LAST], al);
 #pragma unroll
     for (int j = 0; j < NS; ++j)
-      {
-        Tc t[n];
-        lds_read_line<dim, n, LAST>(data + j * STR, p, t);
-        mat_apply<n>(F.V, t, w[j]);
-        lds_write_line_m<dim, n, LAST>(data + j * STR, p, rv[LAST], w[j]);
-      }
+      lds_read_line<dim, n, LAST>(data + j * STR, pv, r[j]);
+    fdm_sweep<n, NS>(F.V, r, [&](int q, const Tc(&v)[NS]) {
+#pragma unroll
+      for (int j = 0; j < NS; ++j)
+        data[j * STR + al[q]] = v[j];
+    });
     __syncthreads();
     if constexpr (dim == 3)
       {
+        lds_line_m<dim, n, 1>(pv, rv[1], al);
 #pragma unroll
         for (int j = 0; j < NS; ++j)
-          {
-            Tc t[n];
-            lds_read_line<dim, n, 1>(data + j * STR, p, t);
-            mat_apply<n>(F.V, t, w[j]);
-            lds_write_line_m<dim, n, 1>(data + j * STR, p, rv[1], w[j]);
-          }
+          lds_read_line<dim, n, 1>(data + j * STR, pv, r[j]);
+        fdm_sweep<n, NS>(F.V, r, [&](int q, const Tc(&v)[NS]) {
+#pragma unroll
+          for (int j = 0; j < NS; ++j)
+            data[j * STR + al[q]] = v[j];
+        });
         __syncthreads();
       }
 #pragma unroll
     for (int j = 0; j < NS; ++j)
-      {
-        Tc t[n];
-        lds_read_line<dim, n, 0>(data + j * STR, p, t);
-        mat_apply<n>(F.V, t, w[j]);
-      }
+      lds_read_line<dim, n, 0>(data + j * STR, pv, r[j]);
 
-    // 5: back stage transform and store (x-lines, mirrored in x)
+    // 5: x sweep, back stage transform and store (x-lines, mirrored in x)
     if (active)
+      fdm_sweep<n, NS>(F.V, r, [&](int q, const Tc(&v)[NS]) {
 #pragma unroll
-      for (int t = 0; t < NS; ++t)
-#pragma unroll
-        for (int i = 0; i < n; ++i)
+        for (int t = 0; t < NS; ++t)
           {
-            Tc s = 0;
+            Tc s = v[0];
+            if constexpr (NS > 1)
+              {
+                s = 0;
 #pragma unroll
-            for (int j = 0; j < NS; ++j)
-              s = fma(F.Tm[t][j], w[j][i], s);
-            dst[t * P.block + cell * nd +
-                L::template off<0>(p, mirror<n>(i, rv[0]))] =
-              (Tout)(NS == 1 ? w[0][i] : s);
+                for (int j = 0; j < NS; ++j)
+                  s = fma(F.Tm[t][j], v[j], s);
+              }
+            dst[t * P.block + x0 + q * xs] = (Tout)s;
           }
+      });
   }
 } // namespace dgops

@@ -215,35 +215,40 @@ namespace dgops
     // factors (see FdmDev::tasks)
     template <typename T>
     void
-    fill_tasks(FdmDev<T> &F, int dim)
+    fill_tasks(FdmDev<T> &F, int dim, int n)
     {
       std::vector<FdmTask<T>> by_nb[5];
       const int               nbd  = F.n_blocks;
       const int               nspb = dim == 3 ? nbd * nbd * nbd : nbd * nbd;
+      const LdsStrides        st   = lds_strides(dim, n);
+      const int               stride[3] = {1, st.x, st.y};
       for (int sb = 0; sb < F.n_stage_blocks; ++sb)
         for (int rb = 0; rb < nspb; ++rb)
           {
             const int  bd[3] = {rb % nbd, (rb / nbd) % nbd,
                                 dim == 3 ? rb / (nbd * nbd) : 0};
             FdmTask<T> tk    = {};
-            const int  js    = F.stage_block_col[sb];
-            const bool sp    = F.stage_block_size[sb] == 2;
-            require(js < 4 && F.n_blocks <= max_n, "FDM task encoding",
-                    DG_ERR_UNSUPPORTED);
-            tk.code  = js | (sp ? 4 : 0);
-            tk.re[0] = F.mre[js];
-            tk.im[0] = sp ? F.mim[js] : (T)0;
-            int nb   = sp ? 1 : 0;
+            int        nb    = 0;
+            const auto pair  = [&](int factor, int delta, T im) {
+              tk.factor[nb] = (uint8_t)factor;
+              tk.delta[nb]  = (int16_t)delta;
+              tk.im[nb]     = im;
+              ++nb;
+            };
+            const int js = F.stage_block_col[sb];
+            int       base = js * st.cell;
+            tk.re[0]       = F.mre[js];
+            if (F.stage_block_size[sb] == 2)
+              pair(0, st.cell, F.mim[js]);
             for (int d = 0; d < dim; ++d)
               {
-                const int  c  = F.block_col[bd[d]];
-                const bool pr = F.block_size[bd[d]] == 2;
-                require(c < 8, "FDM task encoding", DG_ERR_UNSUPPORTED);
-                tk.code |= (c | (pr ? 8 : 0)) << (3 + 4 * d);
+                const int c = F.block_col[bd[d]];
+                base += c * stride[d];
                 tk.re[1 + d] = F.lre[c];
-                tk.im[1 + d] = pr ? F.lim[c] : (T)0;
-                nb += pr ? 1 : 0;
+                if (F.block_size[bd[d]] == 2)
+                  pair(1 + d, stride[d], F.lim[c]);
               }
+            tk.base = (int16_t)base;
             by_nb[nb].push_back(tk);
           }
       int k = 0;
@@ -344,8 +349,8 @@ namespace dgops
         }
       for (int i = 0; i < 4; ++i)
         {
-          fill_tasks(hd[i], op.cfg.dim);
-          fill_tasks(hf[i], op.cfg.dim);
+          fill_tasks(hd[i], op.cfg.dim, n);
+          fill_tasks(hf[i], op.cfg.dim, n);
         }
       op.d_fdm_d.alloc(sizeof(hd));
       op.d_fdm_f.alloc(sizeof(hf));

@@ -36,23 +36,36 @@
 
 namespace dgops
 {
+  // Strides of the y and z coordinates and of the cell in LDS. An even
+  // number of points gets one element of padding per x row: with rows of
+  // 8 (4) values the lanes of a wavefront that read the i-th element of
+  // their x lines share 4 (8) of the 32 double-wide banks, with 9 (5) they
+  // spread over all. Counted over the lanes of a workgroup in all three
+  // directions, the bank cycles per access (1 = no conflict) drop from
+  // 8, 4, 1 to 1, 1, 2 for n = 8 and from 2, 4, 2 to 1, 1, 2 for n = 4
+  // (x, y, z lines, doubles); odd n are conflict free along x already.
+  struct LdsStrides
+  {
+    int x, y, cell;
+  };
+
+  constexpr LdsStrides
+  lds_strides(int dim, int n)
+  {
+    const int x = n % 2 == 1 || (dim == 3 && n == 2) ? n : n + 1;
+    const int y = dim == 3 && n == 2 ? 5 : n * x;
+    return {x, y, dim == 2 ? y : n == 2 ? 12 : n * y};
+  }
+
   template <int dim, int n>
   struct Lay
   {
     static constexpr int nl = dim == 3 ? n * n : n; // lines per cell
     static constexpr int nd = nl * n;               // dofs per cell
 
-    // Strides of the y and z coordinates and of the cell in LDS. An even
-    // number of points gets one element of padding per x row: with rows of
-    // 8 (4) values the lanes of a wavefront that read the i-th element of
-    // their x lines share 4 (8) of the 32 double-wide banks, with 9 (5) they
-    // spread over all. Counted over the lanes of a workgroup in all three
-    // directions, the bank cycles per access (1 = no conflict) drop from
-    // 8, 4, 1 to 1, 1, 2 for n = 8 and from 2, 4, 2 to 1, 1, 2 for n = 4
-    // (x, y, z lines, doubles); odd n are conflict free along x already.
-    static constexpr int sx = n % 2 == 1 || (dim == 3 && n == 2) ? n : n + 1;
-    static constexpr int sy = dim == 3 && n == 2 ? 5 : n * sx;
-    static constexpr int stride = dim == 2 ? sy : n == 2 ? 12 : n * sy;
+    static constexpr int sx     = lds_strides(dim, n).x;
+    static constexpr int sy     = lds_strides(dim, n).y;
+    static constexpr int stride = lds_strides(dim, n).cell;
 
     // LDS offset of point i on line p of direction dir
     template <int dir>

@@ -251,6 +251,56 @@ def test_irk_fdm_is_inverse_of_stage_operator(gpu_lib, s, prec):
         assert err < tol
 
 
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("dim", [2, 3])
+def test_fdm_residual_of_every_degree(gpu_lib, dim, k, prec):
+    """The separable operator on the FDM's result gives the input back, at
+    every degree and stage count (workgroups that end in the middle of their
+    cells, every number of paired eigenvalues). With A = (1 x M..M) X
+    Lambda X^-1, X = T x V..V, the rounding of each of the 2 dim + 2 sweeps
+    and transforms of X Lambda^-1 X^-1 comes back through A with at most
+    cond(T) cond(M) cond(V) per direction times eps."""
+    vel, h, dt = [0.6, -1.0, -0.3][:dim], 0.25, 0.05
+    M, Ks = one_d_matrices(k, 1.0)
+    n, eps = k + 1, (2.2e-16, 1.2e-7)[prec]
+    cond_v = np.linalg.cond(np.linalg.eig(np.linalg.solve(M, Ks[0]))[1])
+    for s in (1, 2, 3, 4):
+        cond_t = np.linalg.cond(np.linalg.eig(irk_coefficients(s)[0])[1]) \
+            if s > 1 else 1
+        tol = (2 * dim + 2) * eps * cond_t * (np.linalg.cond(M) *
+                                              cond_v) ** dim
+        kw = dict(irk_stages=s) if s > 1 else {}
+        c = Cfg(dim=dim, degree=k, refine=2, velocity=vel + [0] * (3 - dim),
+                factor_skew=0.5, precision=prec, **kw)
+        op = AdvectionOperation(c.dg())
+        r = np.random.default_rng(k).standard_normal(op.n_dofs * s)
+        r = r.astype((np.float64, np.float32)[prec]).astype(np.float64)
+        op.set_time(0.0, dt)
+        z = op.initialize_dof_vector(blocks=s)
+        if s > 1:
+            op.precondition_block_jacobi_irk(z, dev(r, op.dtype))
+        else:
+            op.precondition_block_jacobi(z, dev(r, op.dtype))
+        zz = host(z).reshape((s, -1) + (n,) * dim)
+
+        def along(v, mats):
+            for d in range(dim):       # x is the last axis
+                v = np.moveaxis(np.tensordot(v, mats[d], ([-1 - d], [1])),
+                                -1, v.ndim - 1 - d)
+            return v
+        Si = np.linalg.inv(irk_coefficients(s)[0]) if s > 1 else np.eye(1)
+        res = np.tensordot(Si / dt, along(zz, [M] * dim), 1)
+        for d in range(dim):
+            mats = [M] * dim
+            mats[d] = vel[d] / h * Ks[1 if vel[d] < 0 else 0]
+            res += along(zz, mats)
+        err = rel_diff(h ** dim * res.ravel(), r)
+        print(f"fdm residual {dim}D k {k} s {s} prec {prec}: {err:.2e} "
+              f"of {tol:.2e}")
+        assert err < tol
+
+
 def cell_fdm_data(verts, k, dim, velocity):
     """Per cell, from the corners alone: the JxW-weighted mean of the
     reference-space speed J^-1 a over the QGauss(k+1) points and det J at
