@@ -516,6 +516,120 @@ namespace dgops
       }
     aux_inverse_mass(op, op.cfg.precision, dst);
   }
+
+  std::unique_ptr<Operator>
+  create_operator(const dg_config &cfg, hipStream_t stream, DevicePool *pool)
+  {
+    validate(cfg);
+    auto op    = std::make_unique<Operator>();
+    op->cfg    = cfg;
+    op->stream = stream;
+    hip_check(hipGetDevice(&op->device), "hipGetDevice");
+    op->mesh        = make_mesh(mesh_desc(cfg));
+    op->n           = cfg.degree + 1;
+    op->nd          = cfg.dim == 3 ? op->n * op->n * op->n : op->n * op->n;
+    op->n_dofs      = op->mesh.n_cells * op->nd;
+    op->basis       = make_basis(op->n, cfg.use_gl_quad != 0);
+    op->gl_mass_only = !cfg.use_gl_quad && cfg.use_gl_quad_mass;
+    if (cfg.operator_kind == DG_OP_BURGERS)
+      {
+        // QGauss(k(k+1)/2) tables (burgers_solver.cc:234)
+        require(cfg.degree <= (cfg.dim == 3 ? 7 : 4),
+                "Burgers operator: degree 1..7 in 3D, 1..4 in 2D",
+                DG_ERR_UNSUPPORTED);
+        require(cfg.precision == DG_FP64, "Burgers operator: FP64",
+                DG_ERR_UNSUPPORTED);
+        for (int d = 0; d < cfg.dim; ++d)
+          require(cfg.periodic[d],
+                  "Burgers operator: periodic meshes only (the reference "
+                  "has no boundary faces)",
+                  DG_ERR_UNSUPPORTED);
+        BurgersTables T = {};
+        const int     m = cfg.degree * (cfg.degree + 1) / 2;
+        T.m             = m;
+        std::vector<double> gp, gw;
+        gauss_points(m, gp, gw);
+        const auto xl = gauss_lobatto_points_ext(op->n);
+        for (int q = 0; q < m; ++q)
+          {
+            T.wm[q] = gw[q];
+            T.xm[q] = gp[q];
+            for (int i = 0; i < op->n; ++i)
+              {
+                real_ext v, dv;
+                lagrange(xl, i, (real_ext)gp[q], v, dv);
+                T.Sm[q][i] = (double)v;
+                T.Gm[q][i] = (double)dv;
+              }
+          }
+        if (burgers_line_degree(op->n, m))
+          fill_burgers_line(T.line, gp, gw, xl, op->n);
+        op->d_burgers.alloc(sizeof(T));
+        hip_check(hipMemcpy(op->d_burgers.ptr, &T, sizeof(T),
+                            hipMemcpyHostToDevice),
+                  "upload burgers tables");
+      }
+
+    const auto bd = make_dev_basis<double>(op->basis);
+    const auto bf = make_dev_basis<float>(op->basis);
+    if (op->gl_mass_only)
+      {
+        const Basis1D mb  = make_basis(op->n, true);
+        const auto    mbd = make_dev_basis<double>(mb);
+        const auto    mbf = make_dev_basis<float>(mb);
+        op->d_mbasis_d.alloc(sizeof(mbd));
+        op->d_mbasis_f.alloc(sizeof(mbf));
+        hip_check(hipMemcpy(op->d_mbasis_d.ptr, &mbd, sizeof(mbd),
+                            hipMemcpyHostToDevice),
+                  "upload mass basis");
+        hip_check(hipMemcpy(op->d_mbasis_f.ptr, &mbf, sizeof(mbf),
+                            hipMemcpyHostToDevice),
+                  "upload mass basis");
+      }
+    const size_t nb = op->mesh.neighbors.size() * sizeof(int);
+    const size_t nv = op->mesh.cell_vertices.size() * sizeof(double);
+    // small meshes (where the call costs more than the copy): one buffer and
+    // one upload for all four
+    struct Part
+    {
+      DevBuf     &buf;
+      const void *src;
+      size_t      bytes;
+    };
+    const Part parts[] = {{op->d_basis_d, &bd, sizeof(bd)},
+                          {op->d_basis_f, &bf, sizeof(bf)},
+                          {op->d_neighbors, op->mesh.neighbors.data(), nb},
+                          {op->d_vertices, op->mesh.cell_vertices.data(), nv}};
+    const auto aligned = [](size_t b) { return (b + 255) / 256 * 256; };
+    size_t     total   = 0;
+    for (const Part &p : parts)
+      total += aligned(p.bytes);
+    if (total <= size_t(1) << 20)
+      {
+        std::vector<char> staged(total);
+        op->d_setup.pool = pool;
+        op->d_setup.alloc(total);
+        size_t at = 0;
+        for (const Part &p : parts)
+          {
+            std::memcpy(staged.data() + at, p.src, p.bytes);
+            p.buf.view(op->d_setup.as<char>() + at, p.bytes);
+            at += aligned(p.bytes);
+          }
+        hip_check(hipMemcpy(op->d_setup.ptr, staged.data(), total,
+                            hipMemcpyHostToDevice),
+                  "upload basis and mesh");
+      }
+    else
+      for (const Part &p : parts)
+        {
+          p.buf.pool = pool;
+          p.buf.alloc(p.bytes);
+          hip_check(hipMemcpy(p.buf.ptr, p.src, p.bytes, hipMemcpyHostToDevice),
+                    "upload basis and mesh");
+        }
+    return op;
+  }
 } // namespace dgops
 
 using namespace dgops;
@@ -567,91 +681,8 @@ dg_create(const dg_config *cfg, void *stream, dg_operator **out)
   return guard([&] {
     require(cfg && out, "null argument");
     *out = nullptr;
-    validate(*cfg);
-    auto op    = std::make_unique<Operator>();
-    op->cfg    = *cfg;
-    op->stream = (hipStream_t)stream;
-    hip_check(hipGetDevice(&op->device), "hipGetDevice");
-    op->mesh        = make_mesh(mesh_desc(*cfg));
-    op->n           = cfg->degree + 1;
-    op->nd          = cfg->dim == 3 ? op->n * op->n * op->n : op->n * op->n;
-    op->n_dofs      = op->mesh.n_cells * op->nd;
-    op->basis       = make_basis(op->n, cfg->use_gl_quad != 0);
-    op->gl_mass_only = !cfg->use_gl_quad && cfg->use_gl_quad_mass;
-    if (cfg->operator_kind == DG_OP_BURGERS)
-      {
-        // QGauss(k(k+1)/2) tables (burgers_solver.cc:234)
-        require(cfg->degree <= (cfg->dim == 3 ? 7 : 4),
-                "Burgers operator: degree 1..7 in 3D, 1..4 in 2D",
-                DG_ERR_UNSUPPORTED);
-        require(cfg->precision == DG_FP64, "Burgers operator: FP64",
-                DG_ERR_UNSUPPORTED);
-        for (int d = 0; d < cfg->dim; ++d)
-          require(cfg->periodic[d],
-                  "Burgers operator: periodic meshes only (the reference "
-                  "has no boundary faces)",
-                  DG_ERR_UNSUPPORTED);
-        BurgersTables T = {};
-        const int     m = cfg->degree * (cfg->degree + 1) / 2;
-        T.m             = m;
-        std::vector<double> gp, gw;
-        gauss_points(m, gp, gw);
-        const auto xl = gauss_lobatto_points_ext(op->n);
-        for (int q = 0; q < m; ++q)
-          {
-            T.wm[q] = gw[q];
-            T.xm[q] = gp[q];
-            for (int i = 0; i < op->n; ++i)
-              {
-                real_ext v, dv;
-                lagrange(xl, i, (real_ext)gp[q], v, dv);
-                T.Sm[q][i] = (double)v;
-                T.Gm[q][i] = (double)dv;
-              }
-          }
-        if (burgers_line_degree(op->n, m))
-          fill_burgers_line(T.line, gp, gw, xl, op->n);
-        op->d_burgers.alloc(sizeof(T));
-        hip_check(hipMemcpy(op->d_burgers.ptr, &T, sizeof(T),
-                            hipMemcpyHostToDevice),
-                  "upload burgers tables");
-      }
-
-    const auto bd = make_dev_basis<double>(op->basis);
-    const auto bf = make_dev_basis<float>(op->basis);
-    op->d_basis_d.alloc(sizeof(bd));
-    op->d_basis_f.alloc(sizeof(bf));
-    hip_check(hipMemcpy(op->d_basis_d.ptr, &bd, sizeof(bd),
-                        hipMemcpyHostToDevice),
-              "upload basis");
-    hip_check(hipMemcpy(op->d_basis_f.ptr, &bf, sizeof(bf),
-                        hipMemcpyHostToDevice),
-              "upload basis");
-    if (op->gl_mass_only)
-      {
-        const Basis1D mb  = make_basis(op->n, true);
-        const auto    mbd = make_dev_basis<double>(mb);
-        const auto    mbf = make_dev_basis<float>(mb);
-        op->d_mbasis_d.alloc(sizeof(mbd));
-        op->d_mbasis_f.alloc(sizeof(mbf));
-        hip_check(hipMemcpy(op->d_mbasis_d.ptr, &mbd, sizeof(mbd),
-                            hipMemcpyHostToDevice),
-                  "upload mass basis");
-        hip_check(hipMemcpy(op->d_mbasis_f.ptr, &mbf, sizeof(mbf),
-                            hipMemcpyHostToDevice),
-                  "upload mass basis");
-      }
-    const size_t nb = op->mesh.neighbors.size() * sizeof(int);
-    const size_t nv = op->mesh.cell_vertices.size() * sizeof(double);
-    op->d_neighbors.alloc(nb);
-    op->d_vertices.alloc(nv);
-    hip_check(hipMemcpy(op->d_neighbors.ptr, op->mesh.neighbors.data(), nb,
-                        hipMemcpyHostToDevice),
-              "upload neighbors");
-    hip_check(hipMemcpy(op->d_vertices.ptr, op->mesh.cell_vertices.data(), nv,
-                        hipMemcpyHostToDevice),
-              "upload vertices");
-    *out = reinterpret_cast<dg_operator *>(op.release());
+    *out = reinterpret_cast<dg_operator *>(
+      create_operator(*cfg, (hipStream_t)stream, nullptr).release());
   });
 }
 

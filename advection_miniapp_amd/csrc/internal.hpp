@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <array>
 #include <memory>
 #include <stdexcept>
@@ -37,29 +38,132 @@ namespace dgops
 
   void set_last_error(const std::string &msg);
 
-  // device buffer owned by a handle
+  // Device blocks that are given back and taken again without hipFree,
+  // which waits for the device, and hipMalloc. One owner (a server) hands it
+  // to its buffers; a block is given back only when all work on it has
+  // finished. At most `limit` bytes are kept idle, in blocks of at most
+  // max_block; the rest and everything at the end goes to hipFree.
+  struct DevicePool
+  {
+    static constexpr size_t max_block = size_t(16) << 20;
+    struct Block
+    {
+      void  *ptr;
+      size_t bytes;
+      int    device;
+    };
+    std::vector<Block> idle; // oldest first
+    size_t             idle_bytes = 0, limit = 0;
+
+    DevicePool()                              = default;
+    DevicePool(const DevicePool &)            = delete;
+    DevicePool &operator=(const DevicePool &) = delete;
+    ~DevicePool() { trim(0); }
+
+    // an idle block of the current device and of this size in whole pages,
+    // or a new one
+    Block
+    take(size_t b)
+    {
+      Block blk = {nullptr, (std::max<size_t>(b, 1) + 4095) / 4096 * 4096, 0};
+      hip_check(hipGetDevice(&blk.device), "hipGetDevice");
+      for (size_t i = 0; i < idle.size(); ++i)
+        if (idle[i].device == blk.device && idle[i].bytes == blk.bytes)
+          {
+            blk = idle[i];
+            idle.erase(idle.begin() + i);
+            idle_bytes -= blk.bytes;
+            return blk;
+          }
+      if (hipMalloc(&blk.ptr, blk.bytes) != hipSuccess)
+        {
+          (void)hipGetLastError();
+          trim(0);
+          hip_check(hipMalloc(&blk.ptr, blk.bytes), "hipMalloc");
+        }
+      return blk;
+    }
+
+    void
+    give(const Block &b) noexcept
+    {
+      try
+        {
+          if (b.bytes <= max_block && b.bytes <= limit)
+            {
+              idle.push_back(b);
+              idle_bytes += b.bytes;
+              trim(limit);
+              return;
+            }
+        }
+      catch (const std::exception &)
+        {
+        }
+      (void)hipFree(b.ptr);
+    }
+
+    // free the oldest blocks until at most `keep` bytes are idle
+    void
+    trim(size_t keep) noexcept
+    {
+      size_t n = 0;
+      for (; n < idle.size() && idle_bytes > keep; ++n)
+        {
+          idle_bytes -= idle[n].bytes;
+          (void)hipFree(idle[n].ptr);
+        }
+      idle.erase(idle.begin(), idle.begin() + n);
+    }
+  };
+
+  // device buffer owned by a handle, or a part of another one (view)
   struct DevBuf
   {
-    void  *ptr   = nullptr;
-    size_t bytes = 0;
+    void       *ptr    = nullptr;
+    size_t      bytes  = 0;
+    DevicePool *pool   = nullptr; // from and to which, if any
+    bool        owned  = true;
+    int         device = 0; // of a pool's block
     DevBuf() = default;
     DevBuf(const DevBuf &) = delete;
     DevBuf &operator=(const DevBuf &) = delete;
     ~DevBuf() { release(); }
     void release()
     {
-      if (ptr)
-        (void)hipFree(ptr);
+      if (ptr && owned)
+        {
+          if (pool)
+            pool->give({ptr, bytes, device});
+          else
+            (void)hipFree(ptr);
+        }
       ptr   = nullptr;
       bytes = 0;
+      owned = true;
     }
     void alloc(size_t b)
     {
       if (b <= bytes && ptr)
         return;
       release();
+      if (pool)
+        {
+          const DevicePool::Block blk = pool->take(b);
+          ptr                         = blk.ptr;
+          bytes                       = blk.bytes;
+          device                      = blk.device;
+          return;
+        }
       hip_check(hipMalloc(&ptr, b ? b : 8), "hipMalloc");
       bytes = b;
+    }
+    void view(void *p, size_t b)
+    {
+      release();
+      ptr   = p;
+      bytes = b;
+      owned = false;
     }
     template <typename T>
     T *as() const
@@ -108,6 +212,8 @@ namespace dgops
     int            device = 0;
 
     Basis1D basis;
+    // basis tables and mesh arrays; parts of d_setup when they are small
+    DevBuf  d_setup;
     DevBuf  d_basis_d, d_basis_f, d_neighbors, d_vertices;
     // use_gl_quad_mass without use_gl_quad: the mass matrix is integrated
     // with QGaussLobatto(k+1) (its basis in d_mbasis_*), the operator with
@@ -195,6 +301,12 @@ namespace dgops
     }
     void  *solver_vector(size_t idx, size_t bytes);
   };
+
+  // the operator of dg_create; its basis tables and mesh arrays come from
+  // the pool, if there is one
+  std::unique_ptr<Operator> create_operator(const dg_config &cfg,
+                                            hipStream_t      stream,
+                                            DevicePool      *pool);
 
   // kernels launched from host code
   void launch_operator(const Operator &op,

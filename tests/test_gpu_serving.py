@@ -86,6 +86,33 @@ def test_budget_limits_concurrency_and_keeps_results():
         assert err < 1e-14, (r.degree, r.cells_per_direction, err)
 
 
+def test_reused_buffers_give_the_same_results():
+    """Three rounds of the same requests on one server, in another order and
+    under a budget that holds a part of them: buffers of finished requests
+    serve later ones, the results stay bitwise those of a fresh server, and
+    the device memory is free again when the server is gone."""
+    reqs = requests()
+    first, _ = run_server(1 << 34, reqs)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    srv = Server(2 * (3 * 8 * 16 ** 3 * 4 ** 3 + 16 ** 3 * 216 + 40000))
+    kept = []
+    for shift in (0, 4, 7):
+        order = np.roll(np.arange(len(reqs)), shift)
+        ids = {int(i): srv.submit(reqs[i]) for i in order}
+        left = len(ids)
+        while left:
+            left -= srv.step(max_steps=7)[2]
+        for i, rid in ids.items():
+            kept.append((i, srv.take_result(rid)))
+        assert srv.memory() == 0
+    for i, u in kept:
+        assert torch.equal(u, first[i]), i
+    del srv, kept, u
+    torch.cuda.empty_cache()
+    assert torch.cuda.mem_get_info()[0] >= free
+
+
 def test_oversized_request_is_rejected():
     srv = Server(1 << 20)
     r = serve_request(4, 16, [1, 0, 0], [0.5] * 3, 0.1)
