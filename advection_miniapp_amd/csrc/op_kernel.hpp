@@ -619,7 +619,7 @@ namespace dgops
   // weighted with jump; wd is the product of the weights of the line's other
   // coordinates.
   template <int dim, int n, int dir, typename T, bool skew, bool diff,
-            bool local, bool add>
+            bool boundary, bool add>
   __device__ __forceinline__ void
   line_operator(const OpParams       &P,
                 const DevBasis<T>    &B,
@@ -646,14 +646,13 @@ namespace dgops
       {
         const int fc = 2 * dir + s;
         T         up = uplus[fc];
-        if (!local && !diff && P.has_boundary)
+        if (boundary && P.has_boundary)
           {
             // Dirichlet data, evaluated before the launch
             // (boundary_value_kernel)
             const int bi = P.bnd_index[cell * 2 * dim + fc];
             const T   bv =
-              (T)P.bnd_value[(int64_t)(bi >= 0 ? bi : 0) * Lay<dim, n>::nl +
-                             p];
+              (T)P.bnd_value[(int64_t)max(bi, 0) * Lay<dim, n>::nl + p];
             up = bi >= 0 ? bv : up;
           }
         const T an = fan[fc], j = um[s] - up;
@@ -1241,11 +1240,36 @@ namespace dgops
                   }
               }
           }
+        // Dirichlet data of the boundary faces: one component reads those
+        // of all faces here, two rounds of loads; direction by direction a
+        // small mesh waited for six (degree 2, 24x16x8 cells: 6.07 -> 5.36
+        // us). Several components keep to that: the registers of this block
+        // cost them more (degree 4, 32^3 cells, three components: operator
+        // and FDM 206 -> 212 us).
+        constexpr bool BND  = !diff && fin != fin_local;
+        constexpr bool LATE = BND && NC > 1;
+        if constexpr (BND && !LATE)
+          if (P.has_boundary)
+            {
+              int bi[2 * dim];
+              T   bv[2 * dim];
+#pragma unroll
+              for (int f = 0; f < 2 * dim; ++f)
+                bi[f] = P.bnd_index[cell * 2 * dim + f];
+#pragma unroll
+              for (int f = 0; f < 2 * dim; ++f)
+                bv[f] = (T)P.bnd_value[(int64_t)max(bi[f], 0) * nl + p];
+#pragma unroll
+              for (int f = 0; f < 2 * dim; ++f)
+                {
+                  T &u = uplus[0][f];
+                  u    = bi[f] >= 0 ? bv[f] : u;
+                }
+            }
         const T vf    = (T)P.vel_factor[c];
         const T fcell = (T)(-(1. - P.skew) * P.sign) * vf;
         const T fs    = (T)(P.skew * P.sign) * vf;
         const FluxFactors<T> F(P, P.vel_factor[c]);
-        constexpr bool       LOC = fin == fin_local;
         constexpr bool       MASS = fin != fin_inverse_mass;
         const T (&up)[2 * dim] = uplus[NUP > 1 ? c : 0];
         const T (&dp)[2 * dim] = dplus[NUP > 1 ? c : 0];
@@ -1279,7 +1303,7 @@ namespace dgops
               if constexpr (skew)
                 sk[i] = fs * cv[LAST][i];
             }
-          line_operator<dim, n, LAST, T, skew, diff, LOC, MASS>(
+          line_operator<dim, n, LAST, T, skew, diff, LATE, MASS>(
             P, B, F, cell, p, up, dp, fan, uc, g, sk,
             (T)wl[LAST], acc);
           if constexpr (early_ij)
@@ -1348,7 +1372,7 @@ namespace dgops
                 for (int i = 0; i < n; ++i)
                   sk[i] = fs * cvd[i];
               }
-            line_operator<dim, n, 1, T, skew, diff, LOC, true>(
+            line_operator<dim, n, 1, T, skew, diff, LATE, true>(
               P, B, F, cell, p, up, dp, fan, uq, g, sk, (T)wl[1],
               acc);
             lds_write_line<dim, n, 1>(acc_l, p, acc);
@@ -1377,7 +1401,7 @@ namespace dgops
               for (int i = 0; i < n; ++i)
                 sk[i] = fs * cvd[i];
             }
-          line_operator<dim, n, 0, T, skew, diff, LOC, true>(
+          line_operator<dim, n, 0, T, skew, diff, LATE, true>(
             P, B, F, cell, p, up, dp, fan, uq, g, sk, (T)wl[0],
             acc);
         }
