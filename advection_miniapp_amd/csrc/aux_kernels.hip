@@ -916,15 +916,16 @@ namespace dgops
         Lay<dim, n>::template idx<dim - 1>(p, 0, q);
     }
 
-    // one block per cell: w adj(J) a and 1/JxW at the Gauss points
-    // (lexicographic), and w (adj(J) a)_d on the lower face of every
-    // direction, indexed by the line p of direction d that ends on it
-    template <int dim, int n>
+    // one block per cell: w adj(J) a and 1/JxW (or what it is computed from)
+    // at the Gauss points, see TableLay, and w (adj(J) a)_d on the lower face
+    // of every direction, indexed by the line p of direction d that ends on it
+    template <int dim, int n, typename T>
     __global__ void
     geometry_table_kernel(const OpParams P,
                           const DevBasis<double> *__restrict__ B,
-                          double *tab_cell, double *tab_face)
+                          T *tab_cell, T *tab_face)
     {
+      using TL         = TableLay<dim, n, T>;
       constexpr int NV = 1 << dim;
       constexpr int nl = Lay<dim, n>::nl, nd = Lay<dim, n>::nd;
       __shared__ double X[NV * dim];
@@ -932,7 +933,7 @@ namespace dgops
       for (int e = threadIdx.x; e < NV * dim; e += blockDim.x)
         X[e] = P.cell_vertices[cell * NV * dim + e];
       __syncthreads();
-      double *tc = tab_cell + cell * (dim + 1) * nd;
+      T *tc = tab_cell + cell * TL::stride;
       for (int pt = threadIdx.x; pt < nd; pt += blockDim.x)
         {
           const int q[3] = {pt % n, (pt / n) % n,
@@ -947,10 +948,37 @@ namespace dgops
               const int p = d == 0 ? q[1] + n * q[2]
                           : d == 1 ? q[0] + n * q[2]
                                    : q[0] + n * q[1];
-              tc[d * nd + i * nl + p] = cv[d];
+              tc[d * nd + i * nl + p] = (T)cv[d];
             }
-          tc[dim * nd + q[0] * nl + q[1] + n * q[2]] = 1. / jxw;
+          if constexpr (!TL::coef)
+            tc[dim * nd + q[0] * nl + q[1] + n * q[2]] = (T)(1. / jxw);
         }
+      if constexpr (TL::coef)
+        for (int p = threadIdx.x; p < nl; p += blockDim.x)
+          {
+            // det J = j0 . (j1 x j2) with the columns j0 constant and j1, j2
+            // linear along x
+            const int q[2] = {p % n, p / n};
+            double    xi[3] = {0., B->xq[q[0]], B->xq[q[1]]};
+            double    x[3], A[3][3], E[3][3];
+            multilinear_map<dim>(X, xi, x, A);
+            xi[0] = 1.;
+            multilinear_map<dim>(X, xi, x, E);
+            double c[3] = {0., 0., 0.};
+            for (int e = 0; e < 3; ++e)
+              {
+                const int    f = (e + 1) % 3, g = (e + 2) % 3;
+                const double d1f = E[f][1] - A[f][1], d1g = E[g][1] - A[g][1];
+                const double d2f = E[f][2] - A[f][2], d2g = E[g][2] - A[g][2];
+                c[0] += A[e][0] * (A[f][1] * A[g][2] - A[g][1] * A[f][2]);
+                c[1] += A[e][0] * ((A[f][1] * d2g - A[g][1] * d2f) +
+                                   (d1f * A[g][2] - d1g * A[f][2]));
+                c[2] += A[e][0] * (d1f * d2g - d1g * d2f);
+              }
+            const double w = B->w[q[0]] * B->w[q[1]];
+            for (int k = 0; k < 3; ++k)
+              tc[dim * nd + k * nl + p] = (T)(w * c[k]);
+          }
       for (int t = threadIdx.x; t < dim * nl; t += blockDim.x)
         {
           const int d = t / nl, p = t % nl;
@@ -958,7 +986,7 @@ namespace dgops
           face_line_point<dim, n>(d, p, q);
           double an, x[3];
           face_point_data<dim>(P, X, B->xq, B->w, d, 0, q, an, x);
-          tab_face[(cell * dim + d) * nl + p] = -an;
+          tab_face[(cell * dim + d) * nl + p] = (T)-an;
         }
     }
 
@@ -1006,16 +1034,22 @@ namespace dgops
                                       P.vel_const, x);
     }
 
-    template <int dim, int n>
+    template <int dim, int n, typename T>
     void
     launch_geometry_tables(Operator &op, const OpParams &P)
     {
-      const auto *B = op.d_basis_d.as<DevBasis<double>>();
-      if (op.mesh.n_cells > 0)
-        hipLaunchKernelGGL((geometry_table_kernel<dim, n>),
-                           dim3(op.mesh.n_cells), dim3(aux_threads), 0,
-                           op.stream, P, B, op.d_tab_cell[0].as<double>(),
-                           op.d_tab_face[0].as<double>());
+      const int     pi = sizeof(T) == 4 ? 1 : 0;
+      const auto   *B  = op.d_basis_d.as<DevBasis<double>>();
+      const int64_t nc = op.mesh.n_cells;
+      op.d_tab_cell[pi].alloc(sizeof(T) * TableLay<dim, n, T>::stride *
+                              std::max<int64_t>(1, nc));
+      op.d_tab_face[pi].alloc(sizeof(T) * dim * Lay<dim, n>::nl *
+                              std::max<int64_t>(1, nc));
+      if (nc > 0)
+        hipLaunchKernelGGL((geometry_table_kernel<dim, n, T>), dim3(nc),
+                           dim3(aux_threads), 0, op.stream, P, B,
+                           op.d_tab_cell[pi].template as<T>(),
+                           op.d_tab_face[pi].template as<T>());
       hip_check(hipGetLastError(), "geometry tables");
     }
 
@@ -1145,37 +1179,19 @@ namespace dgops
     if (op.tables_ready[pi])
       return;
     aux_boundary_tables(op);
-    const int     dim = op.cfg.dim, n = op.n;
-    const int     nl  = dim == 3 ? n * n : n;
-    const int64_t nc  = op.mesh.n_cells;
-    if (!op.tables_ready[0])
-      {
-        op.d_tab_cell[0].alloc(sizeof(double) * (dim + 1) * op.n_dofs);
-        op.d_tab_face[0].alloc(sizeof(double) * dim * nl *
-                               std::max<int64_t>(1, nc));
-        const OpParams P = op.base_params(0, 1);
+    const int      dim = op.cfg.dim, n = op.n;
+    const OpParams P   = op.base_params(0, 1);
 #define DG_GT(D, N)                                                         \
-  else if (dim == D && n == N) launch_geometry_tables<D, N>(op, P);
-        if (false)
-          ;
-        DG_GT(2, 2) DG_GT(2, 3) DG_GT(2, 4) DG_GT(2, 5) DG_GT(2, 6)
-        DG_GT(2, 7) DG_GT(2, 8) DG_GT(3, 2) DG_GT(3, 3) DG_GT(3, 4)
-        DG_GT(3, 5) DG_GT(3, 6) DG_GT(3, 7) DG_GT(3, 8)
+  else if (dim == D && n == N)                                              \
+    pi == 1 ? launch_geometry_tables<D, N, float>(op, P) :                  \
+              launch_geometry_tables<D, N, double>(op, P);
+    if (false)
+      ;
+    DG_GT(2, 2) DG_GT(2, 3) DG_GT(2, 4) DG_GT(2, 5) DG_GT(2, 6) DG_GT(2, 7)
+    DG_GT(2, 8) DG_GT(3, 2) DG_GT(3, 3) DG_GT(3, 4) DG_GT(3, 5) DG_GT(3, 6)
+    DG_GT(3, 7) DG_GT(3, 8)
 #undef DG_GT
-        op.tables_ready[0] = true;
-      }
-    if (pi == 1)
-      {
-        const int64_t ncell = (dim + 1) * op.n_dofs;
-        const int64_t nface = (int64_t)dim * nl * nc;
-        op.d_tab_cell[1].alloc(sizeof(float) * std::max<int64_t>(1, ncell));
-        op.d_tab_face[1].alloc(sizeof(float) * std::max<int64_t>(1, nface));
-        vec_copy_convert(op, ncell, DG_FP64, op.d_tab_cell[0].ptr, DG_FP32,
-                         op.d_tab_cell[1].ptr);
-        vec_copy_convert(op, nface, DG_FP64, op.d_tab_face[0].ptr, DG_FP32,
-                         op.d_tab_face[1].ptr);
-        op.tables_ready[1] = true;
-      }
+    op.tables_ready[pi] = true;
   }
 
   void

@@ -53,11 +53,11 @@ namespace dgops
     // 3b) and the face neighbours follow from it; -1: read `neighbors`
     int           morton_bits;
     // geometry tables of the tabulated-geometry kernels (scalar type of
-    // the kernel): per cell [dim + 1][nd] = w adj(J) a (dim rows) and
-    // 1/JxW at the Gauss points, each row in the line order of the
-    // direction it is read along (row d along d, row dim along x: point i
-    // of line p at i * nl + p; JxW of the implicit mass term is recomputed
-    // from the corners along the lines); per
+    // the kernel): per cell [dim][nd] = w adj(J) a at the Gauss points and
+    // a row for 1/JxW (TableLay in op_kernel.hpp), each row in the line
+    // order of the direction it is read along (row d along d, row dim along
+    // x: point i of line p at i * nl + p; JxW of the implicit mass term is
+    // recomputed from the corners along the lines); per
     // cell [dim][nl] = w (adj(J) a)_d on the face at xi_d = 0 (normal
     // along +xi_d); per boundary face [nl][1 + dim] (double) = outward
     // a . n dA and the physical point

@@ -351,19 +351,39 @@ namespace dgops
       v[i] = buf[Lay<dim, n>::template loff<dir>(p, i)];
   }
 
-  // row `row` of a cell's geometry table [dim + 1][nd] along line p of the
-  // direction the row is stored in (the direction it is read along: row d
-  // along d, row dim along x), point i at i * nl + p, so that the lanes of
-  // a cell read contiguous memory
+  // Geometry table of a cell: dim rows of nd speeds and the row of 1/JxW of
+  // the inverse mass. The determinant of a trilinear map is quadratic along
+  // a line, so FP64 rows of more than three points hold its coefficients in
+  // the line coordinate times the weight product of the line's other
+  // coordinates instead: 3 values of n, for two multiplications, an estimate
+  // and two Newton steps per point in kernels that are bound by the table's
+  // bytes (MI355X, perturbed cells, before and after: degree 4, 64^3 cells 362
+  // -> 347 us, 32^3 cells degree 5 74 -> 68, 6 122 -> 114, 7 172 -> 158 us;
+  // degree 3, 64^3 cells 175 -> 172). FP32 keeps the values themselves (the sum of three rounded
+  // coefficients would add to their error), and so does 2D (rows of 2n
+  // values, small meshes).
   template <int dim, int n, typename T>
+  struct TableLay
+  {
+    static constexpr bool coef   = dim == 3 && n > 3 && sizeof(T) == 8;
+    static constexpr int  nij    = coef ? 3 : n;
+    static constexpr int  stride =
+      dim * Lay<dim, n>::nd + nij * Lay<dim, n>::nl;
+  };
+
+  // NV values of row `row` of a cell's geometry table along line p of the
+  // direction the row is stored in (the direction it is read along: row d
+  // along d, row dim along x), value i at i * nl + p, so that the lanes of
+  // a cell read contiguous memory
+  template <int dim, int n, typename T, int NV>
   __device__ __forceinline__ void
-  table_line(const T *tab, int64_t cell, int row, int p, T (&v)[n])
+  table_line(const T *tab, int64_t cell, int row, int p, T (&v)[NV])
   {
     constexpr int nd   = Lay<dim, n>::nd;
     constexpr int nl   = Lay<dim, n>::nl;
-    const T      *base = tab + (cell * (dim + 1) + row) * nd;
+    const T      *base = tab + cell * TableLay<dim, n, T>::stride + row * nd;
 #pragma unroll
-    for (int i = 0; i < n; ++i)
+    for (int i = 0; i < NV; ++i)
       v[i] = base[i * nl + p];
   }
 
@@ -1175,7 +1195,8 @@ namespace dgops
     // phase (one component; several components read it per component
     // after their x phase)
     constexpr bool early_ij = geo == geo_table && fin == fin_inverse_mass;
-    T ij_row[early_ij ? n : 1];
+    using TL = TableLay<dim, n, T>;
+    T ij_row[early_ij ? TL::nij : 1];
     if constexpr (UNI)
       {
 #pragma unroll
@@ -1439,6 +1460,21 @@ namespace dgops
 #pragma unroll
                 for (int i = 0; i < n; ++i)
                   ij[i] = B.winv[i] * r;
+              }
+            else if constexpr (TL::coef)
+              {
+                // 1 / (w_i det): the hardware's estimate of the reciprocal
+                // and two Newton steps (~1 ulp, det > 0)
+#pragma unroll
+                for (int i = 0; i < n; ++i)
+                  {
+                    const T x = B.xq[i];
+                    const T d = fma(fma(ij_row[2], x, ij_row[1]), x, ij_row[0]);
+                    T       r = __builtin_amdgcn_rcp(d);
+                    r         = fma(r, fma(-d, r, (T)1), r);
+                    r         = fma(r, fma(-d, r, (T)1), r);
+                    ij[i]     = B.winv[i] * r;
+                  }
               }
             else
 #pragma unroll

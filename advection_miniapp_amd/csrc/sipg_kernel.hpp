@@ -412,7 +412,7 @@ namespace dgops
             }
           else
             {
-              const double *row = tab + cell * (dim + 1) * nd;
+              const double *row = tab + cell * TableLay<dim, n, double>::stride;
               if constexpr (dim == 3)
                 {
                   cv[0] = row[ia * nl + ib + n * i];
