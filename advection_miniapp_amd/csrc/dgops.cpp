@@ -305,7 +305,18 @@ namespace dgops
           throw Error(DG_ERR_UNSUPPORTED,
                       "SIPG on perturbed cells is built in FP64 (the FP32 "
                       "variants need axis-aligned cells)");
-        aux_sipg_general(const_cast<Operator &>(op), P, fin, epi, io);
+        // built in the default tile shape: any other forced one is refused
+        const int cells = op.tile_force_cells;
+        if (cells > 0 && cells != tile_cells(op.cfg.dim, op.n, 0))
+          throw Error(DG_ERR_UNSUPPORTED,
+                      "tile shape of " + std::to_string(cells) +
+                        " cells per workgroup not built for this operator "
+                        "variant");
+        Operator &m     = const_cast<Operator &>(op);
+        m.last_tile     = {0, 0., false};
+        m.last_tile_key = op_key(op.cfg.dim, op.n, nc, 0, geo_table,
+                                 skew ? 1 : 0, diff, fin, epi);
+        aux_sipg_general(m, P, fin, epi, io);
         return;
       }
     // axis-aligned cells with a constant transport speed need no tables

@@ -201,3 +201,24 @@ def test_sipg_perturbed_fp32_and_irk_are_refused(gpu_lib):
         with pytest.raises(L.DgError) as e:
             op.compute_rhs(z, op.initialize_dof_vector())
         assert e.value.code == L.DG_ERR_UNSUPPORTED
+
+
+def test_sipg_perturbed_tile_shapes(gpu_lib):
+    """Perturbed cells are built in the default tile shape: it is reported
+    after a launch, may be forced, and any other one is refused."""
+    from advection_miniapp_amd import _lib as L
+    c = Cfg(dim=3, degree=3, refine=1, perturbation=0.1, operator_kind=1,
+            viscosity=0.05, penalty_factor=16)
+    op = AdvectionOperation(c.dg())
+    src, dst = op.initialize_dof_vector(), op.initialize_dof_vector()
+    op.apply(src, dst, 0.0)
+    shape = op.tile_shape()
+    default = shape["cells_per_workgroup"]
+    assert shape["tuned_ms"] == 0
+    op.set_tile_shape(default)
+    op.apply(src, dst, 0.0)
+    for cells in shape["candidates_ms"]:
+        if cells != default:
+            op.set_tile_shape(cells)
+            with pytest.raises(L.DgError):
+                op.apply(src, dst, 0.0)
