@@ -934,6 +934,12 @@ namespace dgops
         X[e] = P.cell_vertices[cell * NV * dim + e];
       __syncthreads();
       T *tc = tab_cell + cell * TL::stride;
+      // points, lower faces and lines start on successive threads, so that
+      // one pass of the block does them all up to degree 4
+      const auto first = [](int done) {
+        const int b = blockDim.x;
+        return ((int)threadIdx.x + b - done % b) % b;
+      };
       for (int pt = threadIdx.x; pt < nd; pt += blockDim.x)
         {
           const int q[3] = {pt % n, (pt / n) % n,
@@ -954,7 +960,7 @@ namespace dgops
             tc[dim * nd + q[0] * nl + q[1] + n * q[2]] = (T)(1. / jxw);
         }
       if constexpr (TL::coef)
-        for (int p = threadIdx.x; p < nl; p += blockDim.x)
+        for (int p = first(nd + dim * nl); p < nl; p += blockDim.x)
           {
             // det J = j0 . (j1 x j2) with the columns j0 constant and j1, j2
             // linear along x
@@ -979,7 +985,7 @@ namespace dgops
             for (int k = 0; k < 3; ++k)
               tc[dim * nd + k * nl + p] = (T)(w * c[k]);
           }
-      for (int t = threadIdx.x; t < dim * nl; t += blockDim.x)
+      for (int t = first(nd); t < dim * nl; t += blockDim.x)
         {
           const int d = t / nl, p = t % nl;
           int       q[3];
@@ -1125,21 +1131,15 @@ namespace dgops
     const int     nl  = dim == 3 ? n * n : n;
     const int64_t nc  = op.mesh.n_cells;
     // boundary faces in cell order
-    std::vector<int> bidx(std::max<int64_t>(1, nc * 2 * dim), -1);
     std::vector<int> bcell, bface;
     for (int64_t c = 0; c < nc; ++c)
       for (int f = 0; f < 2 * dim; ++f)
         if (op.mesh.neighbors[c * 2 * dim + f] < 0)
           {
-            bidx[c * 2 * dim + f] = (int)bcell.size();
             bcell.push_back((int)c);
             bface.push_back(f);
           }
     const int64_t nb = (int64_t)bcell.size();
-    op.d_bnd_index.alloc(sizeof(int) * bidx.size());
-    hip_check(hipMemcpy(op.d_bnd_index.ptr, bidx.data(),
-                        sizeof(int) * bidx.size(), hipMemcpyHostToDevice),
-              "upload boundary index");
     op.d_tab_bnd.alloc(sizeof(double) * (1 + dim) * nl *
                        std::max<int64_t>(1, nb));
     op.d_bnd_value.alloc(sizeof(double) * nl * std::max<int64_t>(1, nb));

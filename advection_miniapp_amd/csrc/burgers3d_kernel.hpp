@@ -1,5 +1,6 @@
 // Inviscid Burgers right-hand side M^-1(-L(u)) of a 3-component field in 3D
-// for degrees 1..7 (burgers_solver.cc:259-341, the degree a run-time
+// for degrees 1 and 5..7 (2..4: burgers_line_kernel.hpp, whose m^3 points
+// per component fit in LDS) (burgers_solver.cc:259-341, the degree a run-time
 // argument there, :936-938): cell flux u (x) u and the Rusanov face flux
 //   F = 1/2 [(u-.n) u- + (u+.n) u+ + alpha max(|u-.n|, |u+.n|)(u- - u+)]
 // integrated with QGauss(m), m = k(k+1)/2 (burgers_solver.cc:234), and the
@@ -79,8 +80,7 @@ namespace dgops
     static constexpr int UM = m <= 12 ? m : 4;
   };
 
-  // four wavefronts per SIMD where that costs no spills (m <= 6, degree
-  // <= 3: 128 VGPRs with 20 KB of LDS per 3-cell workgroup at degree 3)
+  // four wavefronts per SIMD where that costs no spills (degree 1)
   template <int n, int m, bool cartesian, int epi, int CPB>
   __global__ void __launch_bounds__(CPB * burgers3_threads(n, m))
   __attribute__((amdgpu_waves_per_eu(m <= 6 ? 4 : 1)))

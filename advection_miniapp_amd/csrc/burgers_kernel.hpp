@@ -3,8 +3,9 @@
 //   F = 1/2 [(u-.n) u- + (u+.n) u+ + alpha max(|u-.n|, |u+.n|)(u- - u+)],
 // cell and face integrals with the over-integration rule QGauss(k(k+1)/2)
 // (burgers_solver.cc:234), inverse mass with QGauss(k+1) (:235, :366).
-// The flux is nonlinear and the quadrature differs from the nodal points,
-// so this kernel works point-wise on LDS tensors (one cell per workgroup,
+// The kernel of 2D degree 1 (2..4: burgers_line_kernel.hpp): the flux is
+// nonlinear and the quadrature differs from the nodal points, so it works
+// point-wise on LDS tensors (one cell per workgroup,
 // one thread per quadrature point) instead of the line-per-thread scheme.
 // Faces are element-centric as in op_kernel.hpp: with the cell's own
 // outward normal the plus-side flux of the reference is -F.

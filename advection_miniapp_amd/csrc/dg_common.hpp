@@ -30,7 +30,7 @@ namespace dgops
   struct OpParams
   {
     int64_t       n_cells;
-    const int    *neighbors;     // [cell][2 dim]
+    const int    *neighbors;     // [cell][2 dim]; boundary face b: -1 - b
     const double *cell_vertices; // [cell][2^dim][dim]
     double        h[3];          // cell size when `cartesian`
     double        inv_h[3];      // its reciprocals
@@ -65,7 +65,6 @@ namespace dgops
     const void   *tab_face;
     const double *tab_bnd;
     int           has_boundary; // the mesh has boundary faces
-    const int    *bnd_index; // [cell][2 dim] boundary face id, -1 inside
     const double *bnd_value; // [boundary face][nl] Dirichlet data at sol_time
   };
 

@@ -1,5 +1,6 @@
 // C ABI of the library: handle management, the explicit operator and the
 // low-storage Runge-Kutta integrator, index export, vector operations.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <map>
@@ -336,7 +337,6 @@ namespace dgops
     else
       aux_boundary_tables(m);
     Pk.tab_bnd   = m.d_tab_bnd.as<double>();
-    Pk.bnd_index = m.d_bnd_index.as<int>();
     Pk.bnd_value = m.d_bnd_value.as<double>();
     Pk.has_boundary = m.n_bnd > 0;
     aux_boundary_values(m, Pk);
@@ -597,7 +597,21 @@ namespace dgops
                             hipMemcpyHostToDevice),
                   "upload mass basis");
       }
-    const size_t nb = op->mesh.neighbors.size() * sizeof(int);
+    // the device's neighbour of a boundary face is -1 - its number (in cell
+    // order, as aux_boundary_tables counts them)
+    std::vector<int> numbered;
+    if (std::any_of(op->mesh.neighbors.begin(), op->mesh.neighbors.end(),
+                    [](int c) { return c < 0; }))
+      {
+        numbered  = op->mesh.neighbors;
+        int n_bnd = 0;
+        for (int &c : numbered)
+          if (c < 0)
+            c = -1 - n_bnd++;
+      }
+    const std::vector<int> &neighbors =
+      numbered.empty() ? op->mesh.neighbors : numbered;
+    const size_t nb = neighbors.size() * sizeof(int);
     const size_t nv = op->mesh.cell_vertices.size() * sizeof(double);
     // small meshes (where the call costs more than the copy): one buffer and
     // one upload for all four
@@ -609,7 +623,7 @@ namespace dgops
     };
     const Part parts[] = {{op->d_basis_d, &bd, sizeof(bd)},
                           {op->d_basis_f, &bf, sizeof(bf)},
-                          {op->d_neighbors, op->mesh.neighbors.data(), nb},
+                          {op->d_neighbors, neighbors.data(), nb},
                           {op->d_vertices, op->mesh.cell_vertices.data(), nv}};
     const auto aligned = [](size_t b) { return (b + 255) / 256 * 256; };
     size_t     total   = 0;

@@ -239,10 +239,9 @@ namespace dgops
     // is applied in the kernel)
     DevBuf d_tab_cell[2], d_tab_face[2];
     bool   tables_ready[2] = {false, false};
-    // boundary faces of every geometry mode: index per cell face, a . n dA
-    // and x per face point (built once), Dirichlet data at those points
-    // (refreshed per launch)
-    DevBuf  d_tab_bnd, d_bnd_index, d_bnd_value;
+    // boundary faces of every geometry mode: a . n dA and x per face point
+    // (built once), Dirichlet data at those points (refreshed per launch)
+    DevBuf  d_tab_bnd, d_bnd_value;
     bool    boundary_ready = false;
     int64_t n_bnd          = 0; // boundary faces
 

@@ -670,10 +670,10 @@ namespace dgops
           {
             // Dirichlet data, evaluated before the launch
             // (boundary_value_kernel)
-            const int bi = P.bnd_index[cell * 2 * dim + fc];
+            const int nb = P.neighbors[cell * 2 * dim + fc];
             const T   bv =
-              (T)P.bnd_value[(int64_t)max(bi, 0) * Lay<dim, n>::nl + p];
-            up = bi >= 0 ? bv : up;
+              (T)P.bnd_value[(int64_t)max(~nb, 0) * Lay<dim, n>::nl + p];
+            up = nb < 0 ? bv : up;
           }
         const T an = fan[fc], j = um[s] - up;
         f[s] = fma(an, fma(F.c_own, um[s], F.c_nb * up),
@@ -929,11 +929,10 @@ namespace dgops
 #pragma unroll
             for (int f = 0; f < 2 * dim; ++f)
               {
-                const int bi = P.bnd_index[cell * 2 * dim + f];
+                const int b = NC > 1 ? P.neighbors[cell * 2 * dim + f] : nb[f];
                 const T   an =
-                  (T)P.tab_bnd[((int64_t)(bi >= 0 ? bi : 0) * nl + p) *
-                               (1 + dim)];
-                fan[f] = bi >= 0 ? an : fan[f];
+                  (T)P.tab_bnd[((int64_t)max(~b, 0) * nl + p) * (1 + dim)];
+                fan[f] = b < 0 ? an : fan[f];
               }
           }
     };
@@ -1262,29 +1261,27 @@ namespace dgops
               }
           }
         // Dirichlet data of the boundary faces: one component reads those
-        // of all faces here, two rounds of loads; direction by direction a
-        // small mesh waited for six (degree 2, 24x16x8 cells: 6.07 -> 5.36
-        // us). Several components keep to that: the registers of this block
-        // cost them more (degree 4, 32^3 cells, three components: operator
-        // and FDM 206 -> 212 us).
+        // of all faces here, in one round of loads; direction by direction
+        // a small mesh waited for three (and as many for the face numbers,
+        // before they came with the neighbours; degree 2, 24x16x8 cells:
+        // 6.07 -> 4.96 us). Several components keep to that and read the
+        // neighbours again: the registers cost them more (degree 4, 32^3
+        // cells, three components: operator and FDM 206 -> 212 us; degree 2
+        // 50 -> 54 us).
         constexpr bool BND  = !diff && fin != fin_local;
         constexpr bool LATE = BND && NC > 1;
         if constexpr (BND && !LATE)
           if (P.has_boundary)
             {
-              int bi[2 * dim];
-              T   bv[2 * dim];
+              T bv[2 * dim];
 #pragma unroll
               for (int f = 0; f < 2 * dim; ++f)
-                bi[f] = P.bnd_index[cell * 2 * dim + f];
-#pragma unroll
-              for (int f = 0; f < 2 * dim; ++f)
-                bv[f] = (T)P.bnd_value[(int64_t)max(bi[f], 0) * nl + p];
+                bv[f] = (T)P.bnd_value[(int64_t)max(~nb[f], 0) * nl + p];
 #pragma unroll
               for (int f = 0; f < 2 * dim; ++f)
                 {
                   T &u = uplus[0][f];
-                  u    = bi[f] >= 0 ? bv[f] : u;
+                  u    = nb[f] < 0 ? bv[f] : u;
                 }
             }
         const T vf    = (T)P.vel_factor[c];
