@@ -60,10 +60,10 @@ namespace dgops
     DevicePool &operator=(const DevicePool &) = delete;
     ~DevicePool() { trim(0); }
 
-    // an idle block of the current device and of this size in whole pages,
-    // or a new one
+    // an idle block of the current device and of this size in whole pages
+    // (ptr null: there is none)
     Block
-    take(size_t b)
+    take_idle(size_t b)
     {
       Block blk = {nullptr, (std::max<size_t>(b, 1) + 4095) / 4096 * 4096, 0};
       hip_check(hipGetDevice(&blk.device), "hipGetDevice");
@@ -75,6 +75,16 @@ namespace dgops
             idle_bytes -= blk.bytes;
             return blk;
           }
+      return blk;
+    }
+
+    // such a block, or a new one
+    Block
+    take(size_t b)
+    {
+      Block blk = take_idle(b);
+      if (blk.ptr)
+        return blk;
       if (hipMalloc(&blk.ptr, blk.bytes) != hipSuccess)
         {
           (void)hipGetLastError();
@@ -149,14 +159,23 @@ namespace dgops
       release();
       if (pool)
         {
-          const DevicePool::Block blk = pool->take(b);
-          ptr                         = blk.ptr;
-          bytes                       = blk.bytes;
-          device                      = blk.device;
+          hold(pool->take(b));
           return;
         }
       hip_check(hipMalloc(&ptr, b ? b : 8), "hipMalloc");
       bytes = b;
+    }
+    // alloc, if the pool has an idle block for it
+    void alloc_idle(size_t b)
+    {
+      if (pool && !ptr)
+        hold(pool->take_idle(b));
+    }
+    void hold(const DevicePool::Block &blk)
+    {
+      ptr    = blk.ptr;
+      bytes  = blk.ptr ? blk.bytes : 0;
+      device = blk.device;
     }
     void view(void *p, size_t b)
     {

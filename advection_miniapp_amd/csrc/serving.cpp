@@ -198,14 +198,15 @@ namespace dgops
                              sizeof(DevBasis<float>));
     }
 
-    // idle blocks count against the budget, and no more than idle_limit is
-    // kept: beyond it a solve takes far longer than its allocations
+    // idle blocks count against the budget, `reserve` bytes of which are
+    // about to be allocated, and no more than idle_limit is kept: beyond it
+    // a solve takes far longer than its allocations
     static constexpr int64_t idle_limit = int64_t(128) << 20;
     void
-    bound_pool()
+    bound_pool(int64_t reserve = 0)
     {
-      pool.limit =
-        (size_t)std::max<int64_t>(0, std::min(idle_limit, budget - used));
+      pool.limit = (size_t)std::max<int64_t>(
+        0, std::min(idle_limit, budget - used - reserve));
       pool.trim(pool.limit);
     }
 
@@ -225,6 +226,7 @@ namespace dgops
       q.state    = DG_REQUEST_FAILED;
       q.err_code = code;
       q.err_msg  = "request " + std::to_string(q.id) + " setup: " + msg;
+      bound_pool();
     }
 
     // the tile shape of the request's fused LSRK stage kernel, tuned (or
@@ -256,13 +258,18 @@ namespace dgops
           queue.pop_front();
           try
             {
-              q.handle = reinterpret_cast<dg_operator *>(
-                create_operator(q.cfg, stream, &pool).release());
+              // idle blocks that fit serve as registers; of the others only
+              // what the budget leaves beside this request stays
               for (auto &r : q.reg)
                 {
                   r.pool = &pool;
-                  r.alloc(q.vec_bytes);
+                  r.alloc_idle(q.vec_bytes);
                 }
+              bound_pool(need);
+              q.handle = reinterpret_cast<dg_operator *>(
+                create_operator(q.cfg, stream, &pool).release());
+              for (auto &r : q.reg)
+                r.alloc(q.vec_bytes);
               aux_project(*q.op(), q.reg[0].ptr, 0.);
               q.shape = tuned_shape(q);
             }
@@ -406,12 +413,13 @@ namespace dgops
               continue;
             }
           q.state = DG_REQUEST_DONE;
+          // the pool's share grows first, so that it keeps the blocks
+          used -= 2 * q.vec_bytes + q.op_bytes;
+          bound_pool();
           q.reg[1].release();
           q.reg[2].release();
           dg_destroy(q.handle);
           q.handle = nullptr;
-          used -= 2 * q.vec_bytes + q.op_bytes;
-          bound_pool();
           ++finished;
         }
       active.swap(still);
@@ -540,8 +548,8 @@ dg_server_take_result(dg_server *hs, int64_t id, void *dst)
               "copy result");
     hip_check(hipStreamSynchronize(S.stream), "copy result");
     S.used -= q.vec_bytes;
-    S.reqs.erase(it);
     S.bound_pool();
+    S.reqs.erase(it);
   });
 }
 

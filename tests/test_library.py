@@ -150,3 +150,23 @@ def test_failed_serving_request_is_released_with_its_error():
                                None)
     assert st.value == _lib.DG_REQUEST_UNKNOWN
     assert lib.dg_server_destroy(srv) == 0
+
+
+def test_serving_stays_within_its_budget_during_admission():
+    """tests/cpp/serving_budget (host only: it counts the library's device
+    allocations): requests that follow finished ones of another size find
+    the budget filled with idle buffers, and the memory held never exceeds
+    it; the same request again takes its registers from the idle buffers,
+    and nothing is left when the server is gone. Beyond the budget's own
+    count are the whole-page rounding of four blocks (16 KiB) and one step's
+    launch descriptors (5 stages, 4 solves, under 1 KiB each)."""
+    import os
+    import subprocess
+    tool = os.path.join(os.path.dirname(__file__), "cpp", "serving_budget")
+    assert os.path.exists(tool), "run __graft_entry__.build() first"
+    out = subprocess.run([tool], check=True, capture_output=True,
+                         text=True).stdout
+    budget, peak, again, left = map(int, out.split())
+    assert peak <= budget + 16 * 1024 + 20 * 1024, (peak, budget)
+    assert again <= 1
+    assert left == 0
