@@ -90,6 +90,21 @@ namespace dgops
     int64_t       block;         // stage block size (dofs)
   };
 
+  // LDS stride from cell to cell. Step 3 has the cells of a task on
+  // successive lanes; with an even number of stages an even stride leaves
+  // them few banks (degree 3, four stages: 80 values in 2D, 320 in 3D, two
+  // banks of 32), an odd one all. Four stages on one MI355X, before and
+  // after: 3D degree 1, 64^3 cells 65 -> 40 us in FP64 and 39 -> 24 in FP32;
+  // 2D degree 3, 256^2 cells, FP64 34 -> 26 us. Odd stage counts keep the
+  // stride: their sweeps lose as much as step 3 gains.
+  template <int dim, int n, int NS>
+  constexpr int
+  fdm_cell_stride()
+  {
+    const int s = NS * Lay<dim, n>::stride;
+    return NS % 2 == 0 ? s | 1 : s;
+  }
+
   // offsets of the points of LDS line p of direction dir, in reverse order
   // when `rev`: one start and one step per line
   template <int dim, int n, int dir>
@@ -213,7 +228,6 @@ namespace dgops
   {
     const int tid =
       (int)threadIdx.x - first + ((int)threadIdx.x < first ? blockDim.x : 0);
-    constexpr int STR = Lay<dim, n>::stride;
     const int     t0  = F.task_start[NB];
     const int     nt  = (F.task_start[NB + 1] - t0) * CPB;
     for (int t = tid; t < nt; t += blockDim.x)
@@ -236,8 +250,8 @@ namespace dgops
             delta[b] = tk.delta[b];
             li[b]    = tk.im[b] * m[tk.factor[b]];
           }
-        fdm_block<NB, Tc>(s_data + lc * NS * STR, tk.base, delta, lr, li,
-                          m[4]);
+        fdm_block<NB, Tc>(s_data + lc * fdm_cell_stride<dim, n, NS>(), tk.base,
+                          delta, lr, li, m[4]);
       }
   }
 
@@ -281,9 +295,10 @@ namespace dgops
     constexpr int nd  = L::nd;
     constexpr int CPB = cells_per_block<dim, n>();
     constexpr int STR = L::stride;
+    constexpr int CS  = fdm_cell_stride<dim, n, NS>();
     constexpr int LAST = dim - 1;
 
-    __shared__ Tc s_data[CPB * NS * STR];
+    __shared__ Tc s_data[CPB * CS];
 
     const FdmDev<Tc> &F    = *Fp;
     const int         tid  = threadIdx.x;
@@ -292,7 +307,7 @@ namespace dgops
     const int64_t     cell0 = (int64_t)xcd_block(blockIdx.x, gridDim.x) * CPB;
     const bool        active = lc < CPB && cell0 + lc < P.n_cells;
     const int         lcs    = lc < CPB ? lc : 0;
-    Tc               *data   = s_data + lcs * NS * STR;
+    Tc               *data   = s_data + lcs * CS;
     // idle threads load the last cell and store nothing
     const int64_t     cell   = cell0 + lcs < P.n_cells ? cell0 + lcs :
                                                          P.n_cells - 1;
