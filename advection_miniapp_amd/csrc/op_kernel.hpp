@@ -832,10 +832,14 @@ namespace dgops
     __shared__ double s_X[CPB * NX];
     // several components (IRK stages): their values at the quadrature
     // points wait in LDS between the value phase and the operator phase
-    // (LAST-line layout: every thread writes and reads its own line only)
-    // instead of holding NC lines in registers through the operator phase
+    // instead of holding NC lines in registers through the operator phase.
+    // Every thread writes and reads its own LAST line only, so the points
+    // lie thread by thread: no bank conflicts and no padding, and degree 5
+    // with four stages keeps to four FP64 workgroups per CU
+    // (32^3 cells 353 -> 292 us on one MI355X, 297 -> 238 with uniform
+    // geometry)
     constexpr bool STAGE_LDS = NC > 1;
-    __shared__ T   s_stage[STAGE_LDS ? NC * CPB * STR : 1];
+    __shared__ T   s_stage[STAGE_LDS ? NC * CPB * nd : 1];
     // several components, advection: the neighbour traces of component
     // c are interpolated at the start of its operator phase instead of in
     // the value phase, so that one component's traces are live at a time
@@ -870,7 +874,7 @@ namespace dgops
     T      *fan_l = AN ? s_fan + lcs * 2 * (dim - 1) * nl : s_fan;
     double *X     = s_X + lcs * NX;
     auto    stage_l = [&](int c) -> T * {
-      return s_stage + (STAGE_LDS ? (c * CPB + lcs) * STR : 0);
+      return s_stage + (STAGE_LDS ? c * CPB * nd + tid : 0);
     };
 
     // the cell's own values of the first component are requested first:
@@ -989,7 +993,9 @@ namespace dgops
     T    uqs[STAGE_LDS ? 1 : NC][n];
     auto keep_uq = [&](int c, const T(&v)[n]) {
       if constexpr (STAGE_LDS)
-        lds_write_line<dim, n, LAST>(stage_l(c), p, v);
+#pragma unroll
+        for (int i = 0; i < n; ++i)
+          stage_l(c)[i * CPB * nl] = v[i];
       else
 #pragma unroll
         for (int i = 0; i < n; ++i)
@@ -997,7 +1003,9 @@ namespace dgops
     };
     auto get_uq = [&](int c, T(&v)[n]) {
       if constexpr (STAGE_LDS)
-        lds_read_line<dim, n, LAST>(stage_l(c), p, v);
+#pragma unroll
+        for (int i = 0; i < n; ++i)
+          v[i] = stage_l(c)[i * CPB * nl];
       else
 #pragma unroll
         for (int i = 0; i < n; ++i)
