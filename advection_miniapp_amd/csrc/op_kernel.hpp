@@ -1602,7 +1602,13 @@ namespace dgops
   {
     constexpr bool f64 = sizeof(T) == 8;
     if (geo == geo_analytic)
-      return 1;
+      // FP32 takes 135 registers in 2D at degree 3 and 278 in 3D at degree
+      // 7 on its own: 20.7 -> 17.5 us (256^2 cells) and 50 -> 38 us (16^3)
+      // with one wavefront more; FP64 and the implicit operator at degree 7
+      // spill too much for it
+      return !f64 && dim == 2 && n <= 4                            ? 4 :
+             !f64 && dim == 3 && n == 8 && fin == fin_inverse_mass ? 2 :
+                                                                     1;
     if (diff)
       return 2;
     if (NC > 1 && fin == fin_integrate)
@@ -1615,8 +1621,9 @@ namespace dgops
       return f64 ? (n <= 5 || !skew ? 4 : 2) : (n <= 5 ? 6 : 2);
     if (fin == fin_integrate)
       // 3D degree 4: 126-128 VGPRs with at most 8 spilled, instead of
-      // 132-146 at three
-      return n <= 5 ? 4 : 2;
+      // 132-146 at three; FP32 degree 5: 128 instead of 132, 32^3 cells
+      // with boundary faces 54 -> 51 us
+      return n <= 5 || (!f64 && n == 6) ? 4 : 2;
     return 2;
   }
 
