@@ -916,11 +916,30 @@ namespace dgops
         Lay<dim, n>::template idx<dim - 1>(p, 0, q);
     }
 
-    // one block per cell: w adj(J) a and 1/JxW (or what it is computed from)
-    // at the Gauss points, see TableLay, and w (adj(J) a)_d on the lower face
-    // of every direction, indexed by the line p of direction d that ends on it
+    // cells per workgroup of the table kernel: about a thread per point up
+    // to 3D degree 4, four points per thread above, where one or two cells
+    // leave the last wavefront of each kind half empty
+    constexpr int
+    table_cells(int points)
+    {
+      return (points > aux_threads / 2 ? 4 * aux_threads : aux_threads) /
+             points;
+    }
+
+    // w adj(J) a and 1/JxW (or what it is computed from) at the Gauss
+    // points, see TableLay, and w (adj(J) a)_d on the lower face of every
+    // direction, indexed by the line p of direction d that ends on it.
+    // Bound by the speed and the Jacobian of every point, so the wavefronts
+    // are kept full of one kind of task: points of several small cells
+    // together, then their faces, then their lines, each kind starting on a
+    // wavefront of its own (degree 4: 4 wavefronts of points, 3 of faces and
+    // one of lines for two cells). One MI355X, one cell per workgroup with
+    // the kinds on successive threads and now: degree 1, 64^3 cells 672 ->
+    // 85 us; degree 4, 64^3 cells 1240 -> 843; 32^3 cells, degree 2 94 -> 35,
+    // degrees 5 to 7 201, 253 and 276 -> 147, 228 and 267.
     template <int dim, int n, typename T>
-    __global__ void
+    __global__ void __launch_bounds__(aux_threads)
+    __attribute__((amdgpu_waves_per_eu(4)))
     geometry_table_kernel(const OpParams P,
                           const DevBasis<double> *__restrict__ B,
                           T *tab_cell, T *tab_face)
@@ -928,24 +947,26 @@ namespace dgops
       using TL         = TableLay<dim, n, T>;
       constexpr int NV = 1 << dim;
       constexpr int nl = Lay<dim, n>::nl, nd = Lay<dim, n>::nd;
-      __shared__ double X[NV * dim];
-      const int64_t     cell = blockIdx.x;
-      for (int e = threadIdx.x; e < NV * dim; e += blockDim.x)
-        X[e] = P.cell_vertices[cell * NV * dim + e];
+      constexpr int CPB = table_cells(nd);
+      __shared__ double X[CPB * NV * dim];
+      const int64_t cell0 = (int64_t)blockIdx.x * CPB;
+      const int     nc    = (int)min((int64_t)CPB, P.n_cells - cell0);
+      for (int e = threadIdx.x; e < nc * NV * dim; e += aux_threads)
+        X[e] = P.cell_vertices[cell0 * NV * dim + e];
       __syncthreads();
-      T *tc = tab_cell + cell * TL::stride;
-      // points, lower faces and lines start on successive threads, so that
-      // one pass of the block does them all up to degree 4
+      // first task of this thread after `done` tasks of other kinds
       const auto first = [](int done) {
-        const int b = blockDim.x;
-        return ((int)threadIdx.x + b - done % b) % b;
+        const int at = (done + 63) / 64 * 64 % aux_threads;
+        return ((int)threadIdx.x + aux_threads - at) % aux_threads;
       };
-      for (int pt = threadIdx.x; pt < nd; pt += blockDim.x)
+      for (int e = threadIdx.x; e < nc * nd; e += aux_threads)
         {
+          const int lc = e / nd, pt = e - lc * nd;
           const int q[3] = {pt % n, (pt / n) % n,
                             dim == 3 ? pt / (n * n) : 0};
           double    cv[3], jxw;
-          cell_point_data<dim>(P, X, B->xq, B->w, q, cv, jxw);
+          cell_point_data<dim>(P, X + lc * NV * dim, B->xq, B->w, q, cv, jxw);
+          T *tc = tab_cell + (cell0 + lc) * TL::stride;
           // row d in the line order of direction d (row dim, read along x,
           // in that of x): point i of line p at i * nl + p
           for (int d = 0; d < dim; ++d)
@@ -959,40 +980,57 @@ namespace dgops
           if constexpr (!TL::coef)
             tc[dim * nd + q[0] * nl + q[1] + n * q[2]] = (T)(1. / jxw);
         }
-      if constexpr (TL::coef)
-        for (int p = first(nd + dim * nl); p < nl; p += blockDim.x)
-          {
-            // det J = j0 . (j1 x j2) with the columns j0 constant and j1, j2
-            // linear along x
-            const int q[2] = {p % n, p / n};
-            double    xi[3] = {0., B->xq[q[0]], B->xq[q[1]]};
-            double    x[3], A[3][3], E[3][3];
-            multilinear_map<dim>(X, xi, x, A);
-            xi[0] = 1.;
-            multilinear_map<dim>(X, xi, x, E);
-            double c[3] = {0., 0., 0.};
-            for (int e = 0; e < 3; ++e)
-              {
-                const int    f = (e + 1) % 3, g = (e + 2) % 3;
-                const double d1f = E[f][1] - A[f][1], d1g = E[g][1] - A[g][1];
-                const double d2f = E[f][2] - A[f][2], d2g = E[g][2] - A[g][2];
-                c[0] += A[e][0] * (A[f][1] * A[g][2] - A[g][1] * A[f][2]);
-                c[1] += A[e][0] * ((A[f][1] * d2g - A[g][1] * d2f) +
-                                   (d1f * A[g][2] - d1g * A[f][2]));
-                c[2] += A[e][0] * (d1f * d2g - d1g * d2f);
-              }
-            const double w = B->w[q[0]] * B->w[q[1]];
-            for (int k = 0; k < 3; ++k)
-              tc[dim * nd + k * nl + p] = (T)(w * c[k]);
-          }
-      for (int t = first(nd); t < dim * nl; t += blockDim.x)
+      for (int t = first(CPB * nd); t < nc * dim * nl; t += aux_threads)
         {
-          const int d = t / nl, p = t % nl;
+          const int lc = t / (dim * nl), f = t - lc * dim * nl;
+          const int d = f / nl, p = f % nl;
           int       q[3];
           face_line_point<dim, n>(d, p, q);
           double an, x[3];
-          face_point_data<dim>(P, X, B->xq, B->w, d, 0, q, an, x);
-          tab_face[(cell * dim + d) * nl + p] = (T)-an;
+          face_point_data<dim>(P, X + lc * NV * dim, B->xq, B->w, d, 0, q, an,
+                               x);
+          tab_face[(cell0 + lc) * dim * nl + f] = (T)-an;
+        }
+      if constexpr (TL::coef)
+        {
+          constexpr int before = (CPB * nd + 63) / 64 * 64 + CPB * dim * nl;
+          for (int t = first(before); t < nc * nl; t += aux_threads)
+            {
+              // det J = j0 . (j1 x j2) with the columns j0 constant and j1,
+              // j2 linear along x
+              const int lc = t / nl, p = t - lc * nl;
+              const int q[2] = {p % n, p / n};
+              const double  b = B->xq[q[0]], mb = 1 - b;
+              const double  c = B->xq[q[1]], mc = 1 - c;
+              const double *V = X + lc * NV * dim;
+              double        j0[3], a1[3], a2[3], d1[3], d2[3];
+              for (int e = 0; e < 3; ++e)
+                {
+                  const double x0 = V[e], x1 = V[3 + e], x2 = V[6 + e],
+                               x3 = V[9 + e], x4 = V[12 + e], x5 = V[15 + e],
+                               x6 = V[18 + e], x7 = V[21 + e];
+                  j0[e] = mc * (mb * (x1 - x0) + b * (x3 - x2)) +
+                          c * (mb * (x5 - x4) + b * (x7 - x6));
+                  // at x = 0 and the change to x = 1
+                  a1[e] = mc * (x2 - x0) + c * (x6 - x4);
+                  a2[e] = mb * (x4 - x0) + b * (x6 - x2);
+                  d1[e] = mc * (x3 - x1) + c * (x7 - x5) - a1[e];
+                  d2[e] = mb * (x5 - x1) + b * (x7 - x3) - a2[e];
+                }
+              double k[3] = {0., 0., 0.};
+              for (int e = 0; e < 3; ++e)
+                {
+                  const int f = (e + 1) % 3, g = (e + 2) % 3;
+                  k[0] += j0[e] * (a1[f] * a2[g] - a1[g] * a2[f]);
+                  k[1] += j0[e] * ((a1[f] * d2[g] - a1[g] * d2[f]) +
+                                   (d1[f] * a2[g] - d1[g] * a2[f]));
+                  k[2] += j0[e] * (d1[f] * d2[g] - d1[g] * d2[f]);
+                }
+              const double w = B->w[q[0]] * B->w[q[1]];
+              T *tc = tab_cell + (cell0 + lc) * TL::stride + dim * nd;
+              for (int i = 0; i < 3; ++i)
+                tc[i * nl + p] = (T)(w * k[i]);
+            }
         }
     }
 
@@ -1051,10 +1089,11 @@ namespace dgops
                               std::max<int64_t>(1, nc));
       op.d_tab_face[pi].alloc(sizeof(T) * dim * Lay<dim, n>::nl *
                               std::max<int64_t>(1, nc));
+      constexpr int CPB = table_cells(Lay<dim, n>::nd);
       if (nc > 0)
-        hipLaunchKernelGGL((geometry_table_kernel<dim, n, T>), dim3(nc),
-                           dim3(aux_threads), 0, op.stream, P, B,
-                           op.d_tab_cell[pi].template as<T>(),
+        hipLaunchKernelGGL((geometry_table_kernel<dim, n, T>),
+                           dim3((nc + CPB - 1) / CPB), dim3(aux_threads), 0,
+                           op.stream, P, B, op.d_tab_cell[pi].template as<T>(),
                            op.d_tab_face[pi].template as<T>());
       hip_check(hipGetLastError(), "geometry tables");
     }
