@@ -251,54 +251,96 @@ def test_irk_fdm_is_inverse_of_stage_operator(gpu_lib, s, prec):
         assert err < tol
 
 
+def host_fdm(M, K, Si, vel, h, dt, r, prec, plant=None):
+    """The factorisation X Lambda^-1 X^-1 r that the kernel evaluates, here
+    in complex arithmetic of its precision, r[stage][cell][z, y, x]. With
+    `plant` the block that is paired in every direction is lost ("zero") or
+    its eigenvalues are conjugated ("sign")."""
+    dim, s, n = len(vel), len(Si), len(M)
+    ctype = (np.complex128, np.complex64)[prec]
+
+    def c(a):
+        return np.asarray(a).astype(ctype)
+
+    def along(v, mats):
+        for d in range(dim):           # x is the last axis
+            v = np.moveaxis(np.tensordot(v, c(mats[d]), ([-1 - d], [1])),
+                            -1, v.ndim - 1 - d)
+        return v
+    lam, V = np.linalg.eig(np.linalg.solve(M, K))
+    W, R = np.linalg.solve(V, np.linalg.inv(M) + 0j), np.eye(n)[::-1]
+    mu, T = np.linalg.eig(Si)
+    z = along(np.tensordot(c(np.linalg.inv(T)), c(r), 1),
+              [W @ R if a < 0 else W for a in vel])
+    den = c(mu / dt).reshape((s, 1) + (1,) * dim)
+    for d in range(dim):
+        shape = [n if e == dim - 1 - d else 1 for e in range(dim)]
+        den = den + c(abs(vel[d]) / h * lam).reshape(shape)
+    pair = np.abs(np.abs(lam.imag) - np.max(np.abs(lam.imag))) < 1e-8
+    block = pair
+    for d in range(1, dim):
+        block = np.multiply.outer(block, pair)
+    if plant == "sign":
+        den = np.where(block, den.conj(), den)
+    if plant == "zero":
+        z = np.where(block, 0, z)
+    z = along(z * (c(1 / h ** dim) / den),
+              [R @ V if a < 0 else V for a in vel])
+    return np.tensordot(c(T), z, 1).real.astype(np.float64)
+
+
 @pytest.mark.parametrize("prec", [0, 1])
 @pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 6, 7])
 @pytest.mark.parametrize("dim", [2, 3])
-def test_fdm_residual_of_every_degree(gpu_lib, dim, k, prec):
-    """The separable operator on the FDM's result gives the input back, at
-    every degree and stage count (workgroups that end in the middle of their
-    cells, every number of paired eigenvalues). With A = (1 x M..M) X
-    Lambda X^-1, X = T x V..V, the rounding of each of the 2 dim + 2 sweeps
-    and transforms of X Lambda^-1 X^-1 comes back through A with at most
-    cond(T) cond(M) cond(V) per direction times eps."""
+def test_fdm_of_every_degree(gpu_lib, dim, k, prec):
+    """The FDM at every degree and stage count (workgroups that end in the
+    middle of their cells, every number of paired eigenvalues) against a
+    dense FP64 solve of the separable operator. The factorisation loses up
+    to cond(V)^dim digits, so the bound is the error of the same
+    factorisation on the host in the kernel's precision, times 8 for another
+    order of its sums and products (real pairs instead of complex numbers).
+    A stage count is checked where that bound stays four times below the
+    error of a lost paired block and of one with the wrong sign; single
+    precision has no digits left beyond (3D, degree 7)."""
     vel, h, dt = [0.6, -1.0, -0.3][:dim], 0.25, 0.05
     M, Ks = one_d_matrices(k, 1.0)
-    n, eps = k + 1, (2.2e-16, 1.2e-7)[prec]
-    cond_v = np.linalg.cond(np.linalg.eig(np.linalg.solve(M, Ks[0]))[1])
+    n, checked = k + 1, 0
     for s in (1, 2, 3, 4):
-        cond_t = np.linalg.cond(np.linalg.eig(irk_coefficients(s)[0])[1]) \
-            if s > 1 else 1
-        tol = (2 * dim + 2) * eps * cond_t * (np.linalg.cond(M) *
-                                              cond_v) ** dim
         kw = dict(irk_stages=s) if s > 1 else {}
         c = Cfg(dim=dim, degree=k, refine=2, velocity=vel + [0] * (3 - dim),
                 factor_skew=0.5, precision=prec, **kw)
         op = AdvectionOperation(c.dg())
+        Si = np.linalg.inv(irk_coefficients(s)[0]) if s > 1 else np.eye(1)
         r = np.random.default_rng(k).standard_normal(op.n_dofs * s)
         r = r.astype((np.float64, np.float32)[prec]).astype(np.float64)
+        cells = r.reshape((s, -1) + (n,) * dim)
+        A = np.kron(Si / dt, dense_cell_operator(M, Ks, [0] * dim, h ** dim,
+                                                 1.0, dim)) + \
+            np.kron(np.eye(s), dense_cell_operator(
+                M, Ks, [v / h for v in vel], h ** dim, 0.0, dim))
+        ref = np.linalg.solve(A, np.moveaxis(cells, 1, 0).reshape(
+            op.n_cells, -1).T).T
+        ref = np.moveaxis(ref.reshape((op.n_cells, s, -1)), 0, 1).ravel()
+
+        def host_error(plant=None):
+            return rel_diff(host_fdm(M, Ks[0], Si, vel, h, dt, cells, prec,
+                                     plant).ravel(), ref)
+        tol = 8 * host_error()
+        if 4 * tol > min(host_error("zero"), host_error("sign")):
+            assert prec == 1
+            continue
         op.set_time(0.0, dt)
         z = op.initialize_dof_vector(blocks=s)
         if s > 1:
             op.precondition_block_jacobi_irk(z, dev(r, op.dtype))
         else:
             op.precondition_block_jacobi(z, dev(r, op.dtype))
-        zz = host(z).reshape((s, -1) + (n,) * dim)
-
-        def along(v, mats):
-            for d in range(dim):       # x is the last axis
-                v = np.moveaxis(np.tensordot(v, mats[d], ([-1 - d], [1])),
-                                -1, v.ndim - 1 - d)
-            return v
-        Si = np.linalg.inv(irk_coefficients(s)[0]) if s > 1 else np.eye(1)
-        res = np.tensordot(Si / dt, along(zz, [M] * dim), 1)
-        for d in range(dim):
-            mats = [M] * dim
-            mats[d] = vel[d] / h * Ks[1 if vel[d] < 0 else 0]
-            res += along(zz, mats)
-        err = rel_diff(h ** dim * res.ravel(), r)
-        print(f"fdm residual {dim}D k {k} s {s} prec {prec}: {err:.2e} "
-              f"of {tol:.2e}")
+        err = rel_diff(host(z), ref)
+        print(f"fdm {dim}D k {k} s {s} prec {prec}: {err:.2e} of {tol:.2e}")
         assert err < tol
+        checked += 1
+    if not checked:
+        pytest.skip("single precision has no digits left in this factorisation")
 
 
 def cell_fdm_data(verts, k, dim, velocity):
