@@ -13,6 +13,19 @@ pytestmark = pytest.mark.gpu
 TOL = 1e-12
 
 
+def _coarse(dim, flat=False):
+    # 77 (or 343) cells, without a factor 2, 3 or 5: the last workgroup is a
+    # partial one at every degree (_ragged), and its first cell is not its
+    # last. flat: in 3D one cell along z, its own neighbour on both sides
+    # where z is periodic; else enough cells for inner, perturbed vertices
+    return [7, 11, 1] if dim == 2 or flat else [7, 7, 7]
+
+
+def _ragged(op):
+    cells = op.tile_shape()["cells_per_workgroup"]
+    assert cells > 1 and op.n_cells % cells != 0, (op.n_cells, cells)
+
+
 def _apply(c, seed, t=0.1):
     import torch
     from advection_miniapp_amd import AdvectionOperation
@@ -20,6 +33,7 @@ def _apply(c, seed, t=0.1):
     u = np.random.default_rng(seed).standard_normal(o.n_dofs)
     dst = op.initialize_dof_vector()
     op.apply(torch.as_tensor(u, device="cuda"), dst, t)
+    _ragged(op)
     return dst.cpu().numpy(), o.apply(u, t)
 
 
@@ -27,12 +41,9 @@ def _apply(c, seed, t=0.1):
 @pytest.mark.parametrize("degree", range(1, 8))
 @pytest.mark.parametrize("speed", ["constant", "per point"])
 def test_sipg_every_degree_on_ragged_meshes(dim, degree, speed):
-    # 3 x 5 (x 1) cells: no tile shape divides the cell count at any degree
-    # above 1, and in 3D a periodic direction has a single cell (its own
-    # neighbour on both sides)
     kind = 0 if speed == "constant" else (2 if dim == 2 else 1)
-    c = Cfg(dim=dim, degree=degree, n_coarse=[3, 5, 1], refine=0,
-            hi=[1.0, 1.0, 1.0], velocity_kind=kind,
+    c = Cfg(dim=dim, degree=degree, n_coarse=_coarse(dim, flat=True),
+            refine=0, hi=[1.0, 1.0, 1.0], velocity_kind=kind,
             velocity=[0.7, -0.4, 0.3], operator_kind=1, viscosity=0.05,
             penalty_factor=(degree + 1) ** 2)
     got, ref = _apply(c, 10 * degree + dim)
@@ -43,7 +54,7 @@ def test_sipg_every_degree_on_ragged_meshes(dim, degree, speed):
 @pytest.mark.parametrize("degree", range(1, 8))
 @pytest.mark.parametrize("skew", [0.0, 0.5])
 def test_advection_boundary_faces_on_ragged_meshes(dim, degree, skew):
-    c = Cfg(dim=dim, degree=degree, n_coarse=[3, 5, 1], refine=0,
+    c = Cfg(dim=dim, degree=degree, n_coarse=_coarse(dim), refine=0,
             hi=[1.0, 1.0, 1.0], perturbation=0.1, periodic=[0, 1, 0],
             velocity_kind=2 if dim == 2 else 1, flux_alpha=0.5,
             factor_skew=skew, solution_kind=2,
@@ -81,8 +92,8 @@ def test_stage_operator_with_boundary_faces(dim, degree, stages):
     # stages: the 4-stage table has 7 digits, the oracle computes its own)
     import torch
     from advection_miniapp_amd import AdvectionOperation
-    c = Cfg(dim=dim, degree=degree, n_coarse=[3, 2, 1], refine=0,
-            perturbation=0.1, periodic=[1, 0, 0], factor_skew=0.5,
+    c = Cfg(dim=dim, degree=degree, n_coarse=_coarse(dim, flat=True),
+            refine=0, perturbation=0.1, periodic=[1, 0, 0], factor_skew=0.5,
             velocity_kind=2, solution_kind=2, solution_param=[np.pi, 0.0],
             irk_stages=stages)
     op, o = AdvectionOperation(c.dg()), c.oracle_handle()
@@ -90,6 +101,7 @@ def test_stage_operator_with_boundary_faces(dim, degree, stages):
     op.set_time(0.2, 0.05)
     dst = op.initialize_dof_vector(blocks=stages)
     op.vmult_irk(dst, torch.as_tensor(Z, device="cuda"))
+    _ragged(op)
     assert rel_diff(dst.cpu().numpy(), o.irk_vmult(Z, 0.2, 0.05)) < TOL
 
 
@@ -98,11 +110,11 @@ def test_stage_operator_with_boundary_faces(dim, degree, stages):
 @pytest.mark.parametrize("speed", ["constant", "tabulated"])
 def test_sipg_on_perturbed_ragged_meshes(dim, degree, speed):
     # right-hand side, stage and implicit operator of the general-cell SIPG
-    # kernel; 15 cells fill no workgroup evenly
+    # kernel
     import torch
     from advection_miniapp_amd import AdvectionOperation
     kind = 0 if speed == "constant" else (2 if dim == 2 else 1)
-    kw = dict(dim=dim, degree=degree, n_coarse=[3, 5, 2], refine=0, seed=5,
+    kw = dict(dim=dim, degree=degree, n_coarse=_coarse(dim), refine=0, seed=5,
               perturbation=0.15, velocity_kind=kind, viscosity=0.05,
               velocity=[0.7, -0.4, 0.3], operator_kind=1,
               penalty_factor=(degree + 1) ** 2)
