@@ -34,6 +34,24 @@ CASES = {
                               velocity_kind=2, time_factor=1,
                               final_time=8.0),
     "3d_k7_cart": dict(dim=3, degree=7, refine=1, velocity=[-1, 0.5, 0.25]),
+    # SIPG on perturbed cells (a kernel of its own: with use_gl_quad_mass in
+    # integrate form before the inverse mass), axis-aligned cells
+    "3d_k3_sipg_pert": dict(dim=3, degree=3, n_coarse=[3, 5, 3], refine=0,
+                            perturbation=0.15, velocity=[0.7, -0.4, 0.3],
+                            operator_kind=1, viscosity=0.05,
+                            penalty_factor=16.0),
+    "3d_k4_sipg_pert_cellular": dict(dim=3, degree=4, refine=2,
+                                     perturbation=0.1, velocity_kind=1,
+                                     operator_kind=1, viscosity=0.05,
+                                     penalty_factor=25.0),
+    "2d_k5_sipg_pert_vortex": dict(dim=2, degree=5, refine=3,
+                                   perturbation=0.1, velocity_kind=2,
+                                   time_factor=1, final_time=8.0,
+                                   operator_kind=1, viscosity=0.05,
+                                   penalty_factor=36.0),
+    "3d_k2_sipg_cart": dict(dim=3, degree=2, refine=2,
+                            velocity=[0.7, -0.4, 0.3], operator_kind=1,
+                            viscosity=0.05, penalty_factor=9.0),
 }
 
 SWITCHES = {"gl_quad": dict(use_gl_quad=1),
@@ -92,7 +110,8 @@ def test_inverse_mass_and_projection_match_oracle(gpu_lib, switch):
 
 @pytest.mark.parametrize("switch", sorted(SWITCHES))
 @pytest.mark.parametrize("name", ["3d_k3_pert_cellular",
-                                  "3d_k2_dirichlet_skew"])
+                                  "3d_k2_dirichlet_skew", "3d_k3_sipg_pert",
+                                  "2d_k5_sipg_pert_vortex"])
 def test_perform_stage_matches_oracle(gpu_lib, name, switch):
     c, op, o = make(name, switch)
     rng = np.random.default_rng(3)
