@@ -77,13 +77,13 @@ namespace dgops
     static constexpr int oX  = oF + 9 * m * n;   // [8][3] corners
     static constexpr int size = oX + 24;
     // unroll of the loops over the m points of a line
-    static constexpr int UM = m <= 12 ? m : 4;
+    static constexpr int UM = m == 1 ? 1 : 4;
   };
 
   // four wavefronts per SIMD where that costs no spills (degree 1)
   template <int n, int m, bool cartesian, int epi, int CPB>
   __global__ void __launch_bounds__(CPB * burgers3_threads(n, m))
-  __attribute__((amdgpu_waves_per_eu(m <= 6 ? 4 : 1)))
+  __attribute__((amdgpu_waves_per_eu(m == 1 ? 4 : 1)))
   burgers3_kernel(const OpParams P, const DevBasis<double> *__restrict__ Bd,
                   const BurgersTables *__restrict__ BT,
                   const OpBuffers<double> io)

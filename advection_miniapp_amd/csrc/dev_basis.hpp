@@ -31,16 +31,15 @@ namespace dgops
     T Sinv[max_n][max_n]; // inverse of S [i][q]
     T D[max_n][max_n];    // collocation derivative [q][p]
     T G[max_n][max_n];    // nodal basis derivative at Gauss points [q][i]
-    T l0[max_n], l1[max_n];     // Gauss-Lagrange values at 0 and 1
-    T dl0[max_n], dl1[max_n];   // Gauss-Lagrange derivatives at 0 and 1
     T dphi0[max_n], dphi1[max_n];
     T w[max_n];    // Gauss weights on [0,1]
     T winv[max_n]; // their reciprocals (0 past n)
     T xq[max_n];   // Gauss points on [0,1]
     T xn[max_n]; // Gauss-Lobatto nodes on [0,1]
     EvenOdd<T> eo_S, eo_Sinv, eo_D; // even-odd forms of S, S^-1, D
-    // even and odd parts of l0 and dl0 (l1 is l0 reversed, dl1 is -dl0
-    // reversed) and their middle values: l0 = le + lo, dl0 = de + dd
+    // the Gauss-Lagrange values l0 and derivatives dl0 at 0 (those at 1 are
+    // l0 and -dl0 reversed) as even and odd parts and middle values:
+    // l0 = le + lo, dl0 = de + dd
     T le[max_h], lo[max_h], de[max_h], dd[max_h], lm, dm;
   };
 
@@ -82,10 +81,6 @@ namespace dgops
             d.D[i][j]    = (T)b.D[i][j];
             d.G[i][j]    = (T)b.G[i][j];
           }
-        d.l0[i]    = (T)b.l0[i];
-        d.l1[i]    = (T)b.l1[i];
-        d.dl0[i]   = (T)b.dl0[i];
-        d.dl1[i]   = (T)b.dl1[i];
         d.dphi0[i] = (T)b.dphi0[i];
         d.dphi1[i] = (T)b.dphi1[i];
         d.w[i]     = (T)b.gauss_wts[i];

@@ -305,12 +305,10 @@ namespace dgops
     const int         lc   = tid / nl;
     const int         p    = tid - lc * nl;
     const int64_t     cell0 = (int64_t)xcd_block(blockIdx.x, gridDim.x) * CPB;
-    const bool        active = lc < CPB && cell0 + lc < P.n_cells;
-    const int         lcs    = lc < CPB ? lc : 0;
-    Tc               *data   = s_data + lcs * CS;
-    // idle threads load the last cell and store nothing
-    const int64_t     cell   = cell0 + lcs < P.n_cells ? cell0 + lcs :
-                                                         P.n_cells - 1;
+    const bool        active = cell0 + lc < P.n_cells;
+    Tc               *data   = s_data + lc * CS;
+    // threads past the last cell load it and store nothing
+    const int64_t     cell   = active ? cell0 + lc : P.n_cells - 1;
 
     // 1/dt, |speed| per direction and det J^-1 of the workgroup's cells,
     // read by any thread in step 3

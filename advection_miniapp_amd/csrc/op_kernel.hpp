@@ -208,54 +208,6 @@ namespace dgops
 
   // ---- small register contractions ---------------------------------------
 
-  // out[q] = sum_i M[q][i] in[i]
-  template <int n, typename T>
-  __device__ __forceinline__ void
-  mat_apply(const T (&M)[max_n][max_n], const T (&in)[n], T (&out)[n])
-  {
-#pragma unroll
-    for (int q = 0; q < n; ++q)
-      {
-        T s = M[q][0] * in[0];
-#pragma unroll
-        for (int i = 1; i < n; ++i)
-          s = fma(M[q][i], in[i], s);
-        out[q] = s;
-      }
-  }
-
-  // out[i] = sum_q M[q][i] in[q]
-  template <int n, typename T>
-  __device__ __forceinline__ void
-  mat_apply_t(const T (&M)[max_n][max_n], const T (&in)[n], T (&out)[n])
-  {
-#pragma unroll
-    for (int i = 0; i < n; ++i)
-      {
-        T s = M[0][i] * in[0];
-#pragma unroll
-        for (int q = 1; q < n; ++q)
-          s = fma(M[q][i], in[q], s);
-        out[i] = s;
-      }
-  }
-
-  // out[i] += sum_q M[q][i] in[q]
-  template <int n, typename T>
-  __device__ __forceinline__ void
-  mat_apply_t_add(const T (&M)[max_n][max_n], const T (&in)[n], T (&out)[n])
-  {
-#pragma unroll
-    for (int i = 0; i < n; ++i)
-      {
-        T s = out[i];
-#pragma unroll
-        for (int q = 0; q < n; ++q)
-          s = fma(M[q][i], in[q], s);
-        out[i] = s;
-      }
-  }
-
   // Even-odd products with a centrosymmetric (skew = false) or
   // skew-centrosymmetric (skew = true) matrix M (EvenOdd in dev_basis.hpp):
   // out = M in, or M^T in (transpose), added to out (add). With
@@ -862,17 +814,16 @@ namespace dgops
     const int64_t      cell_t = (int64_t)block * CPB + lc;
     const bool         active = cell_t < P.n_cells;
     const int64_t      cell   = active ? cell_t : P.n_cells - 1;
-    const int          lcs    = lc;
 
-    T      *u_l   = s_u + lcs * STR;
-    T      *acc_l = s_acc + lcs * STR;
-    T      *g0_l  = AN ? s_g0 + lcs * STR : s_g0;
-    T      *g1_l  = (AN && dim == 3) ? s_g1 + lcs * STR : s_g1;
-    T      *sk0_l = (AN && skew) ? s_sk0 + lcs * STR : s_sk0;
-    T      *sk1_l = (AN && skew && dim == 3) ? s_sk1 + lcs * STR : s_sk1;
-    T      *f_l   = s_face + lcs * FSTR;
-    T      *fan_l = AN ? s_fan + lcs * 2 * (dim - 1) * nl : s_fan;
-    double *X     = s_X + lcs * NX;
+    T      *u_l   = s_u + lc * STR;
+    T      *acc_l = s_acc + lc * STR;
+    T      *g0_l  = AN ? s_g0 + lc * STR : s_g0;
+    T      *g1_l  = (AN && dim == 3) ? s_g1 + lc * STR : s_g1;
+    T      *sk0_l = (AN && skew) ? s_sk0 + lc * STR : s_sk0;
+    T      *sk1_l = (AN && skew && dim == 3) ? s_sk1 + lc * STR : s_sk1;
+    T      *f_l   = s_face + lc * FSTR;
+    T      *fan_l = AN ? s_fan + lc * 2 * (dim - 1) * nl : s_fan;
+    double *X     = s_X + lc * NX;
     auto    stage_l = [&](int c) -> T * {
       return s_stage + (STAGE_LDS ? c * CPB * nd + tid : 0);
     };
