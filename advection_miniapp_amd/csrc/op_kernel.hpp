@@ -311,9 +311,11 @@ namespace dgops
   // and two Newton steps per point in kernels that are bound by the table's
   // bytes (MI355X, perturbed cells, before and after: degree 4, 64^3 cells 362
   // -> 347 us, 32^3 cells degree 5 74 -> 68, 6 122 -> 114, 7 172 -> 158 us;
-  // degree 3, 64^3 cells 175 -> 172). FP32 keeps the values themselves (the sum of three rounded
-  // coefficients would add to their error), and so does 2D (rows of 2n
-  // values, small meshes).
+  // degree 3, 64^3 cells 175 -> 172). Tables that stay in the caches do not
+  // gain by it: up to 8^3 cells degrees 3 to 6 are even, and degree 7 takes 2
+  // to 4% more (a second set of kernels would give 0.3 of 8 us back). FP32
+  // keeps the values themselves (the sum of three rounded coefficients would
+  // add to their error), and so does 2D (rows of 2n values, small meshes).
   template <int dim, int n, typename T>
   struct TableLay
   {
@@ -805,12 +807,15 @@ namespace dgops
     const int          tid  = threadIdx.x;
     const int          lc   = tid / nl;
     const int          p    = tid - lc * nl;
-    // threads past the last cell repeat it and store nothing: every load
-    // below is unconditional (a neighbour across a boundary face is read
-    // from the cell itself and replaced by a select). Branches under a
-    // partial exec mask cost moves and split the load batches, and at 250
-    // and more registers the compiler has placed live-range copies before
-    // the mask is restored.
+    // threads past the last cell repeat it and store nothing: no load below
+    // is in a branch of the source's under a part of the lanes (a neighbour
+    // across a boundary face is read from the cell itself and replaced by a
+    // select). Such branches cost moves and split the load batches, and at
+    // 250 and more registers the compiler has placed live-range copies
+    // before the mask is restored. It still makes branches of the selects of
+    // one component's boundary data: with the loads forced out of them (see
+    // needed()) the boundary meshes lost 4 to 9%, the implicit operator up
+    // to 40% by spills.
     const int64_t      cell_t = (int64_t)block * CPB + lc;
     const bool         active = cell_t < P.n_cells;
     const int64_t      cell   = active ? cell_t : P.n_cells - 1;
@@ -1323,10 +1328,10 @@ namespace dgops
             (T)wl[LAST], acc);
           if constexpr (early_ij)
             {
-              // the 1/JxW row of the inverse mass, requested here (the
-              // LAST speed row is dead) so that it arrives during the y
-              // and x phases instead of after them; no extra registers at
-              // the kernel's peak (3D degree 4: 107 VGPRs either way)
+              // the row of the inverse mass, requested here (the LAST speed
+              // row is dead) so that it arrives during the y and x phases
+              // instead of after them, without registers at the kernel's
+              // peak
               __builtin_amdgcn_s_setprio(3);
               table_line<dim, n>(tab_c, cell, dim, p, ij_row);
               __builtin_amdgcn_s_setprio(0);
@@ -1545,7 +1550,10 @@ namespace dgops
   // Wavefronts per SIMD the compiler has to leave room for. Left alone its
   // scheduler hoists the loads of a whole phase (there is no branch to stop
   // at) and takes one or two occupancy steps more than the values need; the
-  // figures are the steps that cost at most a few spilled registers.
+  // figures are the steps that cost at most a few spilled registers. In 2D
+  // they show in the FP32 implicit operator alone (against no figure, 256^2
+  // cells: degree 4 12.7 -> 11.0 us, degrees 1, 2, 5, 7 up to 14% less or
+  // even, degree 6 19.4 -> 21.2); all others, also small meshes, are even.
   template <int dim, int n, int NC, typename T, int geo, bool skew, bool diff,
             int fin>
   constexpr int
@@ -1563,7 +1571,9 @@ namespace dgops
     if (diff)
       return 2;
     if (NC > 1 && fin == fin_integrate)
-      return dim == 3 ? (f64 ? (n <= 2 ? 3 : 2) :
+      // uniform degree 1 in FP64: 128 registers instead of 130, two stages
+      // on 64^3 cells 40.9 -> 37.8 us
+      return dim == 3 ? (f64 ? (n <= 2 ? (geo == geo_uniform ? 4 : 3) : 2) :
                                (n <= 5 ? (geo == geo_table ? 4 : 3) : 2)) :
                         (f64 ? (n <= 4 ? 3 : 2) : (n <= 5 ? 4 : 3));
     if (dim == 2)
