@@ -23,7 +23,7 @@
 // axis-aligned cells 893 -> 421 us; 32^3 perturbed cells 319 -> 207 us;
 // degree 2, 32^3 72 -> 32 us; degree 4, 16^3 204 -> 147 us; 2D degree 3,
 // 128^2 perturbed cells 201 -> 12 us. Bound by LDS and VALU issue together
-// (771 VALU and 81 LDS instructions per wavefront at degree 3). Five waves
+// (845 VALU and 84 LDS instructions per wavefront at degree 3). Five waves
 // per SIMD fit without spills on axis-aligned cells, three on general ones
 // (four spill: 241 us).
 #pragma once

@@ -130,11 +130,11 @@ namespace dgops
   // their share of the test functions' normal derivative is integrated over
   // the face the same way.
   // Bound by LDS and memory latency at two wavefronts per SIMD: degree 3 in
-  // 3D, 32^3 cells, takes 62 us on one MI355X (three at 168 registers spill
-  // and take 120 us). Before, the advection kernel in integrate form, a
-  // diffusion kernel with one point per task and all operands in LDS, and
-  // the inverse mass took 25 + 129 + 16 us: three passes over the vector,
-  // and 2 to 3 LDS reads per product.
+  // 3D, 32^3 cells, takes 53 us on one MI355X in a kernel trace (three
+  // wavefronts at 168 registers spill and take 120 us). Before, the
+  // advection kernel in integrate form, a diffusion kernel with one point
+  // per task and all operands in LDS, and the inverse mass took 25 + 129 +
+  // 16 us: three passes over the vector, and 2 to 3 LDS reads per product.
   template <int dim, int n, bool skew, int fin, int epi>
   __global__ void __launch_bounds__(block_cells(dim == 3 ? n * n : n) *
                                     (dim == 3 ? n * n : n))

@@ -97,8 +97,8 @@ def test_sipg_implicit_vmult_matches_oracle(gpu_lib):
     assert rel_diff(host(dst), o.vmult(u, 0.2, 0.05)) < 1e-12
 
 
-# SIPG on perturbed (non-axis-aligned) cells: advection operator kernel in
-# integrate form + the general-geometry diffusion kernel + inverse mass
+# SIPG on perturbed (non-axis-aligned) cells: one kernel for advection,
+# diffusion and inverse mass on cells of any shape
 PERTURBED = {
     "3d_k3_const": dict(dim=3, k=3, perturbation=0.1, viscosity=0.05),
     "3d_k4_cellular": dict(dim=3, k=4, perturbation=0.15, viscosity=0.02,
