@@ -682,9 +682,9 @@ def time_burgers():
 
 def time_sipg_perturbed():
     """Configuration 3's operator (degree 3, 32^3 cells, a = (1, 0.5,
-    0.25), nu = 1e-3) on cells perturbed by 10% of h: advection kernel in
-    integrate form + general-geometry SIPG kernel + inverse mass (FP64),
-    against the fused apply on the axis-aligned mesh."""
+    0.25), nu = 1e-3) on cells perturbed by 10% of h: the general-geometry
+    SIPG kernel (FP64, one launch), against the apply on the axis-aligned
+    mesh."""
     import math
     import torch
     base = dict(dim=3, degree=3, refine=5, velocity=[1.0, 0.5, 0.25],
@@ -793,7 +793,10 @@ def main():
                    "n_dofs": n, "refine": args.refine},
         "roofline": {"bound": "hbm", "achieved": achieved,
                      "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": achieved / HBM_PEAK_GBS, "traffic": traffic},
+                     "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
+                     "traffic_source": "counters of this kernel in a run of "
+                                       "their own (profiles/apply_3d_k4_"
+                                       "64cube_traffic.json)"},
         "fp64_tflops": APPLY_FLOP_PER_DOF * n / (ms * 1e-3) / 1e12,
         "tile": op.tile,
     }
